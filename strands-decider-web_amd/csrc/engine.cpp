@@ -1020,6 +1020,10 @@ int mnb_forward(ha_mnb* w, int M, const void* a, void* y, void* stream, bool noa
   hipStream_t st = (hipStream_t)stream;
   ha::MnbArgs g = w->args;
   g.M = M; g.a = a; g.y = y;
+  if (ha::mnb_strip_path(g)) {
+    HA_HIP(ha::launch_mnb_strip(g, st));
+    return HA_OK;
+  }
   if (ha::mnb_packed_path(M, g.N, g.K)) {
     HA_HIP(ha::launch_mnb_gemv(g, st));
     return HA_OK;

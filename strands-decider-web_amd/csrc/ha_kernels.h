@@ -120,6 +120,9 @@ struct MnbArgs {
 };
 hipError_t mnb_check(const MnbArgs& a);
 bool mnb_packed_path(int M, int N, int K);  // whether launch_mnb_gemv (packed weights) serves M rows
+bool mnb_strip_takes(const MnbArgs& a);     // whether launch_mnb_strip can run these operands (K, alignment)
+bool mnb_strip_path(const MnbArgs& a);      // whether it serves them
+hipError_t launch_mnb_strip(const MnbArgs& a, hipStream_t s);
 hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s);  // M <= 64 (mnb_packed_path picks up to 48)
 int mnb_gemm_split(int M, int N, int K);  // K ranges the GEMM uses for this shape (1: none, no workspace)
 hipError_t launch_mnb_gemm(const MnbArgs& a, hipStream_t s);  // any M: tiled GEMM, weights dequantised into LDS

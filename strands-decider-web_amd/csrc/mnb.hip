@@ -10,17 +10,18 @@
 //   hold the low two bits as in the 2-bit layout and bit e of word 2 is element e's high bit. One f16 scale per
 //   `group` (32 or 64) values of a row; symmetric w = (q - 2^(bits-1)) * scale, asymmetric w = q * scale + bias.
 //
-// Three implementations, chosen by M (mnb_packed_path) as the reference chooses its kernels by M:
-//   M <= 2   mnb_gemv_lanes_kernel: weight-bandwidth bound. A wave owns 4 output columns, its lanes run along K
-//            over whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
-//   M <= 64  mnb_gemv_kernel: a workgroup owns 16 output columns and its 8 waves split the K blocks; each lane
-//            dequantises a whole packed block into the f16 B operands of v_mfma_f32_16x16x32_f16 (no LDS), the a
-//            rows are the A operand (16 rows per tile, up to 4 tiles share each dequantised operand), and the
-//            waves' partial sums meet in LDS.
-//   above    mnb_gemm_kernel: compute bound. A tiled MFMA GEMM (128 or 256 x 128 workgroup tiles) whose weight
-//            tiles are dequantised on their way into LDS, so the weights stay packed in HBM. With few output tiles
-//            the K range is split over workgroups and mnb_split_sum_kernel adds the fp32 partials in order.
-// All three dequantise with the same f16 arithmetic (dequant8_pk: each weight rounded to f16 once), accumulate in
+// Implementations, chosen by M as the reference chooses its kernels by M:
+//   M <= 2    mnb_gemv_lanes_kernel: weight-bandwidth bound. A wave owns 4 output columns, its lanes run along K
+//             over whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
+//   M <= 384  mnb_strip_kernel (mnb_strip.hip): each wave of a workgroup takes a part of K through LDS of its own.
+//   M <= 64   mnb_gemv_kernel, where the operands do not suit the strip kernel's DMAs (mnb_strip_takes): a workgroup
+//             owns 16 output columns and its 8 waves split the K blocks; each lane dequantises a whole packed block
+//             into the f16 B operands of v_mfma_f32_16x16x32_f16 (no LDS), the a rows are the A operand (16 rows per
+//             tile, up to 4 tiles share each dequantised operand), and the waves' partial sums meet in LDS.
+//   above     mnb_gemm_kernel: compute bound. A tiled MFMA GEMM (128 or 256 x 128 workgroup tiles) whose weight
+//             tiles are dequantised on their way into LDS, so the weights stay packed in HBM. With few output tiles
+//             the K range is split over workgroups and mnb_split_sum_kernel adds the fp32 partials in order.
+// All dequantise with the same f16 arithmetic (each weight rounded to f16 once), accumulate in
 // fp32 and round the output to f16. Results are deterministic: a split K range is summed in a fixed order that
 // depends only on the shape.
 #include <hip/hip_runtime.h>
@@ -31,12 +32,10 @@
 #include <type_traits>
 
 #include "ha_kernels.h"
+#include "mnb_common.h"
 
 namespace ha {
 namespace {
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
 using gptr = const __attribute__((address_space(1))) T*;
@@ -45,8 +44,6 @@ __device__ __forceinline__ gptr<T> gp(const void* p) { return (gptr<T>)(p); }
 
 constexpr int kBlk = 32;       // elements per packed block
 constexpr int kLanesRows = 2;  // up to this many rows: mnb_gemv_lanes_kernel
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 // Elements 8 j .. 8 j + 7 of a packed block (its `BITS` words in registers), dequantised to f16 in the slot order
 // (e0, e4, e1, e5, e2, e6, e3, e7) of the slice: each 32-bit pair holds elements i and i + 4, which one shift and
@@ -87,8 +84,6 @@ __device__ __forceinline__ h8 dequant8_pk(const unsigned* wd, int j, h2 sc, h2 b
 __device__ __forceinline__ h8 perm8(h8 x) {
   return h8{x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7]};
 }
-
-__device__ __forceinline__ h2 splat2(_Float16 v) { return h2{v, v}; }
 
 // y for M <= 16 MT rows. Workgroup: kGW waves, output columns 16 blockIdx.x .. +15; the K blocks go in groups of
 // four, wave w taking groups w, w + kGW, ... Lane (g = lane / 16, c = lane % 16) loads the whole packed block b0 + g
@@ -508,6 +503,12 @@ bool mnb_packed_path(int M, int N, int K) {
   // 12288 x 2048): up to 64 rows the packed-weight kernels are at least as fast as the tiled GEMM on every shape
   // (at 64 rows 10-28 us against 27-71 us).
   return M <= 64;
+}
+
+bool mnb_strip_path(const MnbArgs& a) {
+  // Up to 384 rows the strip kernel is faster than the tiled GEMM on every projection shape (333 rows: 8 - 35 us against
+  // 20 - 43 us); at 512 rows the GEMM wins on 12288 x 2048 (45 against 49 us). One or two rows: the lanes kernel.
+  return a.M > kLanesRows && a.M <= 384 && mnb_strip_takes(a);
 }
 
 hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s) {

@@ -1,0 +1,76 @@
+"""The strip kernel of the MatMulNBits projections (3 to 384 rows) at the edges of its tiles, against the fp64 oracle: one
+and two rows around each count of 16-row tiles, a column count that no tile count divides, K of one half, an odd number
+of halves and more groups than waves, every weight format; rows that keep their bits whatever M is; operands whose
+alignment sends the call to the general kernels."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+import hybrid_attention as ha
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "oracle"))
+import mnb_oracle as mo  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+# max |err| / max |ref|: weights rounded to f16 once (2^-11 each, averaging over K) and an f16 output (2^-11)
+TOL = 2e-3
+
+
+def _weights(N, K, bits, group, asym, seed):
+    rng = np.random.default_rng(seed)
+    words = rng.integers(0, 2 ** 32, (N, K // 32, mo.words_per_block(bits)), dtype=np.uint64).astype(np.uint32)
+    sc = (0.005 + 0.01 * rng.random((N, K // group))).astype(np.float16)
+    bi = ((rng.random((N, K // group)) - 0.5) * 0.1).astype(np.float16) if asym else None
+    return words, sc, bi
+
+
+def _dev(x):
+    import torch
+    return torch.from_numpy(x.view(np.int32) if x.dtype == np.uint32 else x).to("cuda:0")
+
+
+@pytest.mark.parametrize("N,K,bits,group,asym", [
+    (16, 64, 4, 32, False), (1040, 192, 4, 32, True), (2064, 2112, 4, 64, False), (4112, 1152, 4, 64, True),
+    (12304, 128, 4, 32, False), (1040, 192, 3, 32, False), (528, 2176, 3, 64, True), (1040, 1088, 2, 32, True),
+    (16, 128, 2, 64, False)])
+def test_tile_edges(N, K, bits, group, asym):
+    import torch
+    words, sc, bi = _weights(N, K, bits, group, asym, N + K + bits)
+    W = mo.dequant(words, sc, N, K, bits, group, asym, bi)
+    q, s, b = _dev(words), _dev(sc), _dev(bi) if asym else None
+    w = ha.MnbWeight(N, K, q, s, b, bits=bits, group=group, asym=asym)
+    a = ((np.random.default_rng(1).random((385, K)) - 0.5) * 2).astype(np.float16)
+    ad, ref = _dev(a), mo.matmul(a, W)
+    full = None
+    for M in (384, 3, 15, 16, 17, 32, 33, 49, 65, 81, 97, 113, 129, 193, 257, 385):
+        y = torch.full((M + 1, N), 7.0, dtype=torch.float16, device="cuda:0")
+        w.forward(M, ad, y)
+        torch.cuda.synchronize()
+        g = y.cpu().numpy()
+        assert mo.rel_err(g[:M].astype(np.float64), ref[:M]) < TOL, M
+        assert (g[M] == 7.0).all(), "row past M written (M = %d)" % M
+        if full is None:
+            full = g
+        elif M < 384 and K % 64 == 0 and (group == 32 or K % 128 == 0):
+            assert np.array_equal(g[:M].view(np.uint16), full[:M].view(np.uint16)), "bits of a row depend on M = %d" % M
+    w.close()
+
+
+@pytest.mark.parametrize("bits,off_q,off_s", [(4, 4, 0), (4, 0, 2), (3, 4, 2)])
+def test_unaligned_operands(bits, off_q, off_s):
+    import torch
+    N, K, M = 272, 256, 40
+    words, sc, _ = _weights(N, K, bits, 32, False, bits + off_q)
+    qb = torch.zeros(words.size + 4, dtype=torch.int32, device="cuda:0")
+    sb = torch.zeros(sc.size + 4, dtype=torch.float16, device="cuda:0")
+    qb[off_q // 4:off_q // 4 + words.size] = _dev(words).reshape(-1)
+    sb[off_s // 2:off_s // 2 + sc.size] = _dev(sc).reshape(-1)
+    w = ha.MnbWeight(N, K, qb.data_ptr() + off_q, sb.data_ptr() + off_s, None, bits=bits)
+    a = ((np.random.default_rng(2).random((M, K)) - 0.5) * 2).astype(np.float16)
+    y = torch.empty(M, N, dtype=torch.float16, device="cuda:0")
+    w.forward(M, _dev(a), y)
+    torch.cuda.synchronize()
+    assert mo.rel_err(y.double().cpu().numpy(), mo.matmul(a, mo.dequant(words, sc, N, K, bits))) < TOL
+    w.close()
