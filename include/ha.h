@@ -103,7 +103,7 @@ typedef struct ha_forward_opts {
                       computed on. Implies a wait, like layer_ms */
   int debug_unpublished_waits; /* test only, 0 otherwise. No counterpart in the reference. 1: every bounded
                       cross-workgroup wait of this call (the paired form's tile-set wait, the split form's
-                      packed-state wait, the split-key attention merge) waits for a value no workgroup of it
+                      packed-state wait, the split-key attention merge, a short attention call's maxima) waits for a value no workgroup of it
                       publishes, for a few polls each, then goes on; every kernel still ends, the outputs are
                       undefined, and the failure is reported as HA_ERR_DEVICE (exercises that path from the host) */
 } ha_forward_opts;

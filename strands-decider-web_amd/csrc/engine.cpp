@@ -85,14 +85,14 @@ struct Scratch {
     size_t bytes = 0;
   };
   int device = 0;
-  Buf img, seq_raw, seq_cnt, gqa_part, zeros, duo_ring, sync_flags;
+  Buf img, seq_raw, seq_cnt, gqa_part, gqa_rows, gqa_marks, zeros, duo_ring, sync_flags;
   unsigned sync_epoch = 0;  // the progress counters' epoch of the last launch that used them (they start at zero)
-  unsigned gqa_epoch = 0;   // the split-GQA slot marks' epoch of the last launch (the marks start at zero)
+  unsigned gqa_epoch = 0;   // the GQA marks' epoch of the last launch (the marks start at zero)
   // the engines holding this set (guarded by g_live_mu); all of them run on one stream, so their calls never overlap
   std::vector<const ha_engine*> holders;
   ~Scratch() {
     (void)hipSetDevice(device);
-    for (Buf* b : {&img, &seq_raw, &seq_cnt, &gqa_part, &zeros, &duo_ring, &sync_flags})
+    for (Buf* b : {&img, &seq_raw, &seq_cnt, &gqa_part, &gqa_rows, &gqa_marks, &zeros, &duo_ring, &sync_flags})
       if (b->p) (void)hipFree(b->p);
   }
 };
@@ -138,8 +138,8 @@ struct ha_engine {
   // images [B][H][img_chunks] of the split form (allocated when a call can use that form), the sequential
   // form's raw outputs [B][H][kSegRows][DV] and counters [B][H], split-GQA partials [gqa_part_slots]
   std::shared_ptr<Scratch> scratch;
-  size_t need_zeros = 0, need_img = 0, need_seq_raw = 0, need_seq_cnt = 0, need_gqa = 0, need_duo_ring = 0,
-         need_sync_flags = 0;
+  size_t need_zeros = 0, need_img = 0, need_seq_raw = 0, need_seq_cnt = 0, need_gqa = 0, need_gqa_rows = 0,
+         need_gqa_marks = 0, need_duo_ring = 0, need_sync_flags = 0;
   int img_chunks = 0, duo_slots = 0;
   int gqa_split = 0, gqa_part_slots = 0;
   hipEvent_t ev[2] = {nullptr, nullptr};
@@ -308,6 +308,7 @@ int take_device_error(ha_engine* e) {
   std::string what;
   if (v & ha::kErrDuoWait) what += " a paired-form consumer gave up waiting for a tile set;";
   if (v & ha::kErrSplitWait) what += " a split-form output workgroup gave up waiting for a packed state;";
+  if (v & ha::kErrGqaRows) what += " a short-call attention tile gave up waiting for the row maxima of earlier tiles;";
   if (v & ha::kErrGqaMerge) what += " a split-key attention merge gave up waiting for its pieces;";
   if (what.empty()) what = " unknown code " + std::to_string(v) + ";";
   return fail(HA_ERR_DEVICE, "device error in an earlier kernel of this engine (its outputs are undefined):" +
@@ -472,6 +473,10 @@ int ha_create(const ha_config* cfg, int device, ha_engine** out) {
       e->need_gqa = slots * ha::gqa_part_slot_bytes();
       if ((rc = grow(e->scratch->gqa_part, e->need_gqa))) return bail(rc);
     }
+    e->need_gqa_rows = ha::gqa_rows_bytes((int)B * c.HK, c.max_ctx);
+    e->need_gqa_marks = ha::gqa_rows_marks((int)B * c.HK, c.max_ctx) * sizeof(unsigned);
+    if ((rc = grow(e->scratch->gqa_rows, e->need_gqa_rows)) || (rc = grow(e->scratch->gqa_marks, e->need_gqa_marks)))
+      return bail(rc);
     if (hipMemcpy(e->rope, rope.data(), rope.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(HA_ERR_DEVICE, "hipMemcpy rope failed"));
   }
@@ -506,7 +511,8 @@ int ha_set_stream(ha_engine* e, void* stream) {
     int rc;
     if ((rc = grow(s->zeros, e->need_zeros)) || (rc = grow(s->seq_raw, e->need_seq_raw)) ||
         (rc = grow(s->seq_cnt, e->need_seq_cnt)) || (rc = grow(s->sync_flags, e->need_sync_flags)) ||
-        (rc = grow(s->gqa_part, e->need_gqa)) || (rc = grow(s->img, split_by_shape(c) ? e->need_img : 0)) ||
+        (rc = grow(s->gqa_part, e->need_gqa)) || (rc = grow(s->gqa_rows, e->need_gqa_rows)) ||
+        (rc = grow(s->gqa_marks, e->need_gqa_marks)) || (rc = grow(s->img, split_by_shape(c) ? e->need_img : 0)) ||
         (rc = grow(s->duo_ring, paired_by_shape(c) ? e->need_duo_ring : 0)))
       return rc;
     std::lock_guard<std::mutex> lock(g_live_mu);
@@ -534,6 +540,7 @@ int ha_share_scratch(ha_engine* e, ha_engine* holder) {
   if ((rc = grow(to.zeros, e->need_zeros)) || (rc = grow(to.img, from.img.bytes ? e->need_img : 0)) ||
       (rc = grow(to.seq_raw, e->need_seq_raw)) ||
       (rc = grow(to.seq_cnt, e->need_seq_cnt)) || (rc = grow(to.gqa_part, e->need_gqa)) ||
+      (rc = grow(to.gqa_rows, e->need_gqa_rows)) || (rc = grow(to.gqa_marks, e->need_gqa_marks)) ||
       (rc = grow(to.duo_ring, from.duo_ring.bytes ? e->need_duo_ring : 0)) ||
       (rc = grow(to.sync_flags, e->need_sync_flags)))
     return rc;
@@ -717,11 +724,14 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       a.in = layer_in[i]; a.out = layer_out[i]; a.qw = l.qn; a.kw = l.kn; a.rope = e->rope;
       a.K = l.K; a.V = l.V;
       a.split = e->gqa_split; a.part_slots = e->gqa_part_slots; a.part = static_cast<float*>(sc.gqa_part.p);
-      if (a.split > 0) {
+      a.rows = sc.gqa_rows.p; a.row_marks = static_cast<unsigned*>(sc.gqa_marks.p);
+      const bool rows = ha::gqa_rows_takes(a);
+      if (a.split > 0 || rows) {
         // a fresh mark per launch; if the counter wraps, the marks (and partials) are cleared first
         if (++sc.gqa_epoch == 0) {
           HA_HIP(hipStreamSynchronize(st));
-          HA_HIP(hipMemset(sc.gqa_part.p, 0, sc.gqa_part.bytes));
+          if (sc.gqa_part.p) HA_HIP(hipMemset(sc.gqa_part.p, 0, sc.gqa_part.bytes));
+          HA_HIP(hipMemset(sc.gqa_marks.p, 0, sc.gqa_marks.bytes));
           sc.gqa_epoch = 1;
         }
         a.epoch = sc.gqa_epoch;
@@ -729,7 +739,7 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       // the merge waits for marks equal to this launch's epoch: epoch + 1 is never written by it
       a.wait = wait;
       if (unpublished) a.wait.skew = 1u;
-      hipError_t he = ha::launch_gqa(a, st);
+      hipError_t he = rows ? ha::launch_gqa_rows(a, st) : ha::launch_gqa(a, st);
       if (he != hipSuccess) return fail(HA_ERR_DEVICE, "layer " + std::to_string(i) + " attention launch: " + hipGetErrorString(he));
       if (per_layer) HA_HIP(hipEventRecord(e->mev[i], st));
     } else if (per_layer) {  // HA_ADAPTER: no token mixer, nothing to run

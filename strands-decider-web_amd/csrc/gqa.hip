@@ -24,109 +24,25 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "gqa_common.h"
 #include "ha_kernels.h"
 
 namespace ha {
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef float f16v __attribute__((ext_vector_type(16)));
-
-template <typename T>
-using gptr = const __attribute__((address_space(1))) T*;
-template <typename T>
-__device__ __forceinline__ gptr<T> gp(const void* p) { return (gptr<T>)(p); }
-template <typename T>
-__device__ __forceinline__ __attribute__((address_space(1))) T* gpw(void* p) { return (__attribute__((address_space(1))) T*)(p); }
-
-constexpr int kHD = 256, kBQ = 32, kBK = 64;
+constexpr int kBQ = 32;
 constexpr int kEP = 136;  // row pitch (floats) of the epilogue staging area: rows r and r + 4 sit 32 banks apart
 // two K + V^T tile buffers; after the tile loop, each wave's 32 x 128 f32 epilogue staging area
 constexpr int kTileBytes = kBK * kHD * 2;  // one K tile or one V^T tile (f16)
 // LDS: two (K, V^T) tile buffers; after the tile loop, each wave's 32 x 128 f32 epilogue staging area
 constexpr size_t kAttnLds = 4 * (size_t)kTileBytes > sizeof(float) * 8 * 32 * kEP ? 4 * (size_t)kTileBytes
                                                                                   : sizeof(float) * 8 * 32 * kEP;
-constexpr float kRescale = 8.0f;    // log2 headroom before the reference max is raised
 
 // An identity the compiler cannot see through: lane indices re-derived from it on every tile keep the address
 // arithmetic built on them inside the loop instead of hoisted out of it (and spilled).
 __device__ __forceinline__ int opaque(int x) {
   asm volatile("" : "+v"(x));
   return x;
-}
-
-__device__ __forceinline__ f4 ld4(gptr<float> p) { return *(gptr<f4>)(p); }
-__device__ __forceinline__ f4 ld4(gptr<_Float16> p) {
-  const h4 x = *(gptr<h4>)(p);
-  return f4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
-}
-__device__ __forceinline__ void store4(__attribute__((address_space(1))) float* p, const f4& v) {
-  *(__attribute__((address_space(1))) f4*)(p) = v;
-}
-__device__ __forceinline__ void store4(__attribute__((address_space(1))) _Float16* p, const f4& v) {
-  *(__attribute__((address_space(1))) h4*)(p) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-}
-
-__device__ __forceinline__ f4 lds4(const float* p) { return *reinterpret_cast<const f4*>(p); }
-
-// Orders a wave's LDS writes before its later reads of other lanes' entries (no workgroup barrier).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// max / sum of x over lanes l and l ^ 32: v_permlane32_swap hands every lane both values (in an order that depends
-// on the half, which neither a max nor a two-term sum sees)
-__device__ __forceinline__ void both_halves(float x, float& u, float& v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
-  u = __builtin_bit_cast(float, (unsigned)r[0]);
-  v = __builtin_bit_cast(float, (unsigned)r[1]);
-}
-__device__ __forceinline__ float max_halves(float x) {
-  float u, v;
-  both_halves(x, u, v);
-  return fmaxf(u, v);
-}
-__device__ __forceinline__ float sum_halves(float x) {
-  float u, v;
-  both_halves(x, u, v);
-  return u + v;
-}
-
-__device__ __forceinline__ float sigmoid(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
-
-template <typename T>
-__device__ __forceinline__ void load8f(gptr<T> p, float* o);
-template <>
-__device__ __forceinline__ void load8f<float>(gptr<float> p, float* o) {
-  const f4 x = *(gptr<f4>)(p), y = *(gptr<f4>)(p + 4);
-  o[0] = x[0]; o[1] = x[1]; o[2] = x[2]; o[3] = x[3]; o[4] = y[0]; o[5] = y[1]; o[6] = y[2]; o[7] = y[3];
-}
-template <>
-__device__ __forceinline__ void load8f<_Float16>(gptr<_Float16> p, float* o) {
-  const h8 x = *(gptr<h8>)(p);
-#pragma unroll
-  for (int i = 0; i < 8; i++) o[i] = (float)x[i];
-}
-
-// Sum over the 64 lanes of a wave without LDS: row rotations inside each 16-lane row, then v_permlane16_swap
-// (rows 2r <-> 2r+1) and v_permlane32_swap (halves). Every lane ends with the same bits (each step adds two values
-// that the lanes it pairs see in the other order).
-template <int kCtrl>
-__device__ __forceinline__ float dpp(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float wave_sum64(float v) {
-  v += dpp<0x128>(v);  // row_ror:8
-  v += dpp<0x124>(v);  // row_ror:4
-  v += dpp<0x122>(v);  // row_ror:2
-  v += dpp<0x121>(v);  // row_ror:1
-  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
-  v = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-  return sum_halves(v);
 }
 
 // K rows and V^T columns for rows [t0, t0 + 64) of one (sequence, KV head). Wave w takes rows kKvRows w ..
@@ -160,24 +76,12 @@ __global__ __launch_bounds__(64 * kKvWaves) void gqa_kv_kernel(GqaArgs a) {
     x[r] = ld4(row + (size_t)kh * kHD + 4 * lane);
     vv[r] = ld4(row + (size_t)a.HK * kHD + (size_t)kh * kHD + 4 * lane);
   }
-  const bool rot = lane < 16;  // dims 0 .. 63 (RD = 64)
-  const int ri = 4 * (lane & 7);
+  const int ri = 2 * (lane & 7);
   __syncthreads();  // RoPE rows staged
 #pragma unroll
   for (int r = 0; r < kKvRows; r++) {
     const int t = t0 + kKvRows * wave + r, pos = a.P + min(t, a.L - 1);
-    const float ss = wave_sum64((x[r][0] * x[r][0] + x[r][1] * x[r][1]) + (x[r][2] * x[r][2] + x[r][3] * x[r][3]));
-    const float inv = rsqrtf(ss / kHD + 1e-6f);
-    f4 k = x[r] * inv * kw;
-    f4 pk;
-#pragma unroll
-    for (int c = 0; c < 4; c++) pk[c] = dpp<0x128>(k[c]);  // lane l ^ 8: row_ror:8 within each 16-lane row
-    if (rot) {
-      const f4 cs0 = rope_l[kKvRows * wave + r][ri >> 1], cs1 = rope_l[kKvRows * wave + r][(ri >> 1) + 1];
-      const float cs[4] = {cs0[0], cs0[2], cs1[0], cs1[2]}, sn[4] = {cs0[1], cs0[3], cs1[1], cs1[3]};
-#pragma unroll
-      for (int c = 0; c < 4; c++) k[c] = lane < 8 ? k[c] * cs[c] - pk[c] * sn[c] : k[c] * cs[c] + pk[c] * sn[c];
-    }
+    const f4 k = key_row(x[r], kw, rope_l[kKvRows * wave + r][ri], rope_l[kKvRows * wave + r][ri + 1], lane);
     if (t < a.L)
       *(__attribute__((address_space(1))) h4*)(gpw<_Float16>(a.K) + kvb + (size_t)pos * kHD + 4 * lane) =
           h4{(_Float16)k[0], (_Float16)k[1], (_Float16)k[2], (_Float16)k[3]};
@@ -218,9 +122,6 @@ constexpr int kWaves = 8;
 // after every piece in the grid, wait for the marks of their block's pieces and read the partials with sc1 loads.
 // Each XCD dispatches its blocks in order, so it starts merge workgroups only once all of its pieces are out:
 // pieces never wait, so every mark is eventually written, and each wait is bounded besides.
-constexpr int kCacheSc1 = 16;  // cache-policy operand of buffer instructions: device-coherent (sc1)
-typedef int i4v __attribute__((ext_vector_type(4)));
-typedef int i2v __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ unsigned* part_marks(const GqaArgs& a) {
   return reinterpret_cast<unsigned*>(a.part + (size_t)a.part_slots * 4 * kRows * (kHD + 2));
 }
@@ -393,8 +294,8 @@ __global__ __launch_bounds__(64 * kWaves) void gqa_attn_kernel(GqaArgs a, int pe
                                        (__attribute__((address_space(3))) void*)(vb + (size_t)ins * 512), 16, 0, 0);
     }
   };
-  // kIdleHalf (calls of at most 32 rows, as in a decode step, where every block's second half holds no row of the
-  // call): that half's waves copy every tile and the first half's waves none, which takes the copies off the path of
+  // kIdleHalf (calls of at most 32 rows of batches too large for gqa_rows.hip, where every block's second half holds no
+  // row of the call): that half's waves copy every tile and the first half's waves none, which takes the copies off the path of
   // the waves that compute
   // Longer calls: waves 0..3 (which always hold rows) copy every tile and waves 4..7 none, which staggers the two
   // waves of each SIMD a little (one starts a tile's MFMAs while the other still issues copies).

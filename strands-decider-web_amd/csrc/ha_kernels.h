@@ -17,6 +17,7 @@ namespace ha {
 constexpr unsigned kErrDuoWait = 1u;    // paired form: a consumer gave up waiting for a tile set
 constexpr unsigned kErrSplitWait = 2u;  // split form: an output workgroup gave up waiting for a packed state
 constexpr unsigned kErrGqaMerge = 4u;   // split-key GQA: a merge workgroup gave up waiting for its pieces
+constexpr unsigned kErrGqaRows = 8u;    // short-call GQA: a tile's workgroup gave up waiting for earlier tiles' maxima
 constexpr int kWaitPolls = 1 << 16;
 struct WaitCheck {
   unsigned* err = nullptr;  // host-visible error word (system-scope stores), or nullptr
@@ -77,13 +78,22 @@ struct GqaArgs {
   int part_slots;
   float* part;               // [slots][4][64][HD] unnormalised O, then [slots][4][64][2] (reference max, sum), then
                              // [slots] u32 epoch marks
-  unsigned epoch;            // this launch's mark, >= 1 and different from every earlier launch's on `part`
+  unsigned epoch;            // this launch's mark, >= 1 and different from every earlier launch's on `part` or `row_marks`
+  void* rows;                // short calls: scratch of gqa_rows_bytes(), or nullptr
+  unsigned* row_marks;       // short calls: gqa_rows_marks() marks
   WaitCheck wait;            // the merge workgroups' bounded wait for their pieces
 };
 
 // Slots of partial results the split GQA path needs for any call on a context of at most max_ctx positions.
 size_t gqa_part_slots(int pairs, int max_ctx, int split);
 size_t gqa_part_slot_bytes();
+// Short calls (at most gqa_rows_max(pairs) rows a sequence): every key tile on a workgroup of its own, then every slice of
+// output dims. Needs scratch for any such call on a context of at most max_ctx positions.
+int gqa_rows_max(int pairs);
+size_t gqa_rows_bytes(int pairs, int max_ctx);
+size_t gqa_rows_marks(int pairs, int max_ctx);
+bool gqa_rows_takes(const GqaArgs& a);
+hipError_t launch_gqa_rows(const GqaArgs& a, hipStream_t s);
 
 // Copy the raw rows [dst_first, P + L) (dst_first >= s0 - (KC-1)) of every sequence from (tail, in) into
 // `tail_out` ([B][tail_cap][stride]); only the conv channels [0, C) and the a/b columns are kept.

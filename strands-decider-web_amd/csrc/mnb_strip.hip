@@ -27,25 +27,13 @@
 #include <algorithm>
 
 #include "ha_kernels.h"
+#include "lds_dma.h"
 #include "mnb_common.h"
 
 namespace ha {
 namespace {
 
 constexpr int kSW = 8;  // waves of a workgroup
-
-// LDS DMA, written out so that the compiler does not wait for it before unrelated LDS reads: lane l's bytes land at
-// lds + 16 l (dwordx4) or lds + 4 l (dword). The kernel's own waits order these. m0, the DMA's LDS base, is a register
-// the compiler reserves and does not preserve across asm; no compiler-generated code in these kernels keeps a value
-// in it (tests/test_strip_guards.py checks the assembly).
-__device__ __forceinline__ void dma16(unsigned lds, unsigned voff, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
-               "v"(voff), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(unsigned lds, unsigned voff, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
-               "v"(voff), "s"(base) : "memory", "m0");
-}
 
 // A wave's LDS stage: a rows, packed words, scales (, biases) of one 64-k half; at the end its partial sums.
 template <int BITS, bool ASYM, int MT, int NT>

@@ -1,4 +1,4 @@
-"""Guard on the compiled gfx950 code of mnb_strip.hip: its LDS DMAs set m0, a register the compiler reserves and does not
+"""Guard on the compiled gfx950 code of the files whose LDS DMAs are written out (lds_dma.h): a DMA sets m0, a register the compiler reserves and does not
 preserve across asm, right before the instruction. Sound only while every m0 reference is the asm's own set."""
 import os
 import re
@@ -12,12 +12,13 @@ HIPCC = "/opt/rocm/bin/hipcc"
 pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is missing")
 
 
-def test_m0_is_written_only_by_the_dma_asm(tmp_path):
-    out = tmp_path / "strip.s"
+@pytest.mark.parametrize("name", ["mnb_strip.hip", "gqa_rows.hip"])
+def test_m0_is_written_only_by_the_dma_asm(tmp_path, name):
+    out = tmp_path / "out.s"
     r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                         "-packed-fp32-ops", "-I" + os.path.join(ROOT, "include"),
                         "-I" + os.path.join(ROOT, "strands-decider-web_amd", "csrc"), "-x", "hip", "-S",
-                        "--cuda-device-only", os.path.join(ROOT, "strands-decider-web_amd", "csrc", "mnb_strip.hip"),
+                        "--cuda-device-only", os.path.join(ROOT, "strands-decider-web_amd", "csrc", name),
                         "-o", str(out)], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stderr
     code = [l for l in (l.strip() for l in out.read_text().splitlines()) if l and not l.startswith((";", "."))]
