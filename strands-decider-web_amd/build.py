@@ -17,14 +17,13 @@ LIB = os.path.join(HERE, "libha.so")
 NAPI_OUT = os.path.join(HERE, "js", "ha_napi.node")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["engine.cpp", "gdn_seq.hip", "gdn_chunk.hip", "gdn_duo.hip", "gdn_split.hip", "gqa.hip", "gqa_rows.hip", "tail.hip", "mnb.hip", "mnb_strip.hip", "torso.hip"]
+SOURCES = ["engine.cpp", "gdn_seq.hip", "gdn_chunk.hip", "gdn_duo.hip", "gdn_split.hip", "gqa.hip", "tail.hip", "mnb.hip", "torso.hip"]
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 # Per-source additions. -amdgpu-mfma-vgpr-form keeps MFMA accumulators in VGPRs: the state passes scale their fp32
-# accumulators on the VALU every chunk, which with AGPR accumulators costs a read and a write-back per element; the
-# short-call attention's products follow loads and rescales the same way.
-FILE_FLAGS = {"gdn_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "gqa_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# accumulators on the VALU every chunk, which with AGPR accumulators costs a read and a write-back per element.
+FILE_FLAGS = {"gdn_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd, verbose):

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(64 * kWaves) void gqa_attn_kernel(GqaArgs a, int pe
                                        (__attribute__((address_space(3))) void*)(vb + (size_t)ins * 512), 16, 0, 0);
     }
   };
-  // kIdleHalf (calls of at most 32 rows of batches too large for gqa_rows.hip, where every block's second half holds no
+  // kIdleHalf (calls of at most 32 rows of batches too large for gqa_rows.h, where every block's second half holds no
   // row of the call): that half's waves copy every tile and the first half's waves none, which takes the copies off the path of
   // the waves that compute
   // Longer calls: waves 0..3 (which always hold rows) copy every tile and waves 4..7 none, which staggers the two
@@ -711,3 +711,5 @@ hipError_t launch_gqa(const GqaArgs& a, hipStream_t s) {
 }
 
 }  // namespace ha
+
+#include "gqa_rows.h"

@@ -1,4 +1,4 @@
-// Shared by the full-attention kernels (gqa.hip, gqa_rows.hip), gfx950.
+// Shared by the full-attention kernels (gqa.hip, gqa_rows.h), gfx950.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -1,4 +1,4 @@
-// Full attention of a short call (a decode step, a resumed question), gfx950: the same arithmetic as gqa.hip, row for row
+// Full attention of a short call (a decode step, a resumed question), gfx950, compiled with gqa.hip: the same arithmetic as gqa.hip, row for row
 // and bit for bit, in two launches that put every key tile and every slice of output dims on a workgroup of its own.
 //
 // A short call has one or two 32-row query groups per (sequence, KV head), so gqa_attn_kernel has a handful of workgroups
@@ -20,6 +20,7 @@
 // lowest unfinished block is always resident and waits for finished ones: every wait ends, and each is bounded besides.
 // Measured, f16 rows, us a call, before -> now: 61 rows after 1531 (1 sequence) 61 -> 25; one row after 1536 (8 sequences)
 // 56 -> 28 (scores 15.8, values 12.3), after 3000 93 -> 47; 64 rows of an empty context 26 -> 20.
+#pragma once
 #include <algorithm>
 
 #include "gqa_common.h"
@@ -27,6 +28,7 @@
 #include "lds_dma.h"
 
 namespace ha {
+namespace gqa_rows {
 namespace {
 
 constexpr int kG = 32;           // query rows of a group
@@ -548,6 +550,7 @@ hipError_t launch(const GqaArgs& a, hipStream_t s) {
 }
 
 }  // namespace
+}  // namespace gqa_rows
 
 // The longest call taken, rows a sequence. gqa_attn_kernel has one workgroup per 64 rows and pair (pieces of 8 tiles in
 // engines of one or two pairs), so it catches up as rows and pairs fill the chip; the lines lie where it does. Measured at
@@ -556,11 +559,11 @@ hipError_t launch(const GqaArgs& a, hipStream_t s) {
 int gqa_rows_max(int pairs) { return pairs <= 2 ? 256 : pairs <= 16 ? 128 : pairs <= 32 ? 64 : 0; }
 
 size_t gqa_rows_marks(int pairs, int max_ctx) {
-  return (size_t)pairs * ((gqa_rows_max(pairs) + kG - 1) / kG) * ((max_ctx + kBK - 1) / kBK);
+  return (size_t)pairs * ((gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG) * ((max_ctx + kBK - 1) / kBK);
 }
 size_t gqa_rows_bytes(int pairs, int max_ctx) {
-  const size_t groups = (gqa_rows_max(pairs) + kG - 1) / kG, halves = 2 * (size_t)((max_ctx + kBK - 1) / kBK);
-  return pairs * groups * 4 * halves * kUnitBytes;
+  const size_t groups = (gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG, halves = 2 * (size_t)((max_ctx + kBK - 1) / kBK);
+  return pairs * groups * 4 * halves * gqa_rows::kUnitBytes;
 }
 
 // (HD, RD, heads per pair, LT: as launch_gqa checks them)
@@ -571,10 +574,10 @@ bool gqa_rows_takes(const GqaArgs& a) {
 
 hipError_t launch_gqa_rows(const GqaArgs& a, hipStream_t s) {
   if (!gqa_rows_takes(a) || a.epoch == 0 || a.P + a.L > a.LT) return hipErrorInvalidValue;
-  if (a.split > 0 && (a.LT / kBK + a.split - 1) / a.split > kMaxPieces) return hipErrorInvalidValue;
+  if (a.split > 0 && (a.LT / kBK + a.split - 1) / a.split > gqa_rows::kMaxPieces) return hipErrorInvalidValue;
   // maxima are addressed by 32-bit byte offsets
-  if ((size_t)rows_layout(a).units * kMUnit > 0x7fffffff) return hipErrorInvalidValue;
-  return a.dtype == 0 ? launch<float>(a, s) : launch<_Float16>(a, s);
+  if ((size_t)gqa_rows::rows_layout(a).units * gqa_rows::kMUnit > 0x7fffffff) return hipErrorInvalidValue;
+  return a.dtype == 0 ? gqa_rows::launch<float>(a, s) : gqa_rows::launch<_Float16>(a, s);
 }
 
 }  // namespace ha

@@ -1,7 +1,7 @@
 // LDS DMA written out, gfx950: the compiler would otherwise wait for every DMA in flight before any LDS read, and for
 // the loads issued after it too. Lane l's bytes, from base + voff, land at lds + 16 l (dwordx4) or lds + 4 l (dword); the
 // kernel's own waits (vmcnt) order them. m0, the DMA's LDS base, is a register the compiler reserves and does not preserve
-// across asm: sound while no compiler-generated code of the file keeps a value in it (tests/test_strip_guards.py checks
+// across asm: sound while no compiler-generated code of the kernels that use these keeps a value in it (tests/test_strip_guards.py checks
 // the assembly).
 #pragma once
 #include <hip/hip_runtime.h>

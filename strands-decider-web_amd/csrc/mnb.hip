@@ -13,7 +13,7 @@
 // Implementations, chosen by M as the reference chooses its kernels by M:
 //   M <= 2    mnb_gemv_lanes_kernel: weight-bandwidth bound. A wave owns 4 output columns, its lanes run along K
 //             over whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
-//   M <= 384  mnb_strip_kernel (mnb_strip.hip): each wave of a workgroup takes a part of K through LDS of its own.
+//   M <= 384  mnb_strip_kernel (mnb_strip.h): each wave of a workgroup takes a part of K through LDS of its own.
 //   M <= 64   mnb_gemv_kernel, where the operands do not suit the strip kernel's DMAs (mnb_strip_takes): a workgroup
 //             owns 16 output columns and its 8 waves split the K blocks; each lane dequantises a whole packed block
 //             into the f16 B operands of v_mfma_f32_16x16x32_f16 (no LDS), the a rows are the A operand (16 rows per

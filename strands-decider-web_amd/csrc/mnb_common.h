@@ -1,4 +1,4 @@
-// Weight decoding shared by the MatMulNBits kernels (mnb.hip, mnb_strip.hip), gfx950.
+// Weight decoding shared by the MatMulNBits kernels (mnb.hip, mnb_strip.h), gfx950.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -1,4 +1,4 @@
-// MatMulNBits projection of a few hundred rows or less, gfx950: y[M][N] = a[M][K] x W^T (formats: mnb.hip).
+// MatMulNBits projection of a few hundred rows or less, gfx950, compiled with torso.hip: y[M][N] = a[M][K] x W^T (formats: mnb.hip).
 //
 // Bound: moving a. Each workgroup needs all of its rows of a, so M x K x 2 bytes pass through the L2 once per column
 // tile; the packed weights (0.56 bytes each) are read once or twice. A wave cannot load its MFMA operands from a
@@ -22,6 +22,7 @@
 //   12288 x 2048   7.7 -> 5.9  13.3->6.7  25.8->9.4   22.8->10.2  26.4->14.0  35.2->25.1
 //   2048 x 6144    7.7 -> 6.3  13.9->6.5  24.9->7.7   22.6->8.7   23.9->9.4   24.9->14.7
 //   2048 x 2048    4.4 -> 4.4  5.9 ->4.4  9.8 ->4.5   13.8->4.7   14.6->4.9   16.6->6.5
+#pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,6 +32,7 @@
 #include "mnb_common.h"
 
 namespace ha {
+namespace strip {
 namespace {
 
 constexpr int kSW = 8;  // waves of a workgroup
@@ -189,17 +191,22 @@ hipError_t launch_one(const MnbArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Tile counts a format is built for. 4-bit weights are what the exporter writes; the other widths get fewer shapes.
+// Tile counts a format is built for: all for what the exporter writes (4 bits, groups of 32, symmetric), fewer shapes for
+// the others.
+template <int BITS, int GROUP, bool ASYM>
+constexpr bool kEveryTile = BITS == 4 && GROUP == 32 && !ASYM;
+bool every_tile(const MnbArgs& a) { return a.bits == 4 && a.group == 32 && !a.asym; }
 template <int BITS, int GROUP, bool ASYM>
 hipError_t launch_fmt(const MnbArgs& a, int mt, int nt, hipStream_t s) {
 #define HA_STRIP(MT, NT) \
   if (mt == MT && nt == NT) return launch_one<BITS, GROUP, ASYM, MT, NT>(a, s);
-#define HA_STRIP4(MT) HA_STRIP(MT, 1) HA_STRIP(MT, 2) HA_STRIP(MT, 3) HA_STRIP(MT, 4)
-  HA_STRIP4(1) HA_STRIP4(2) HA_STRIP4(4)
-  if constexpr (BITS == 4) {
-    HA_STRIP4(3) HA_STRIP4(5) HA_STRIP4(6) HA_STRIP(8, 1) HA_STRIP(8, 2) HA_STRIP(8, 3)
+#define HA_STRIP3(MT) HA_STRIP(MT, 1) HA_STRIP(MT, 2) HA_STRIP(MT, 3)
+  HA_STRIP3(1) HA_STRIP3(2) HA_STRIP3(4)
+  if constexpr (kEveryTile<BITS, GROUP, ASYM>) {
+    HA_STRIP3(3) HA_STRIP3(5) HA_STRIP3(6) HA_STRIP3(8)
+    HA_STRIP(1, 4) HA_STRIP(2, 4) HA_STRIP(3, 4) HA_STRIP(4, 4) HA_STRIP(5, 4) HA_STRIP(6, 4)
   }
-#undef HA_STRIP4
+#undef HA_STRIP3
 #undef HA_STRIP
   return hipErrorInvalidValue;
 }
@@ -209,19 +216,19 @@ hipError_t launch_fmt(const MnbArgs& a, int mt, int nt, hipStream_t s) {
 // workgroups a round, over the rounds that needs, and of those the least rounds x (mt + nt + 2). Measured choices
 // (M, N, K: mt x nt us, next best): 61, 2048, 6144: 2 x 1 8.0, 3 x 1 9.0; 61, 12288, 2048: 4 x 3 9.9, 2 x 3 10.4;
 // 128, 5120, 2048: 3 x 4 8.9, 4 x 3 9.1; 192, 8256, 2048: 4 x 4 18.0, 3 x 3 18.7.
-void pick_tiles(int M, int N, int bits, int* mt, int* nt) {
+void pick_tiles(int M, int N, bool every, int* mt, int* nt) {
   const int tm = (M + 15) / 16, tn = N / 16;
   int best = 1 << 30;
   *mt = *nt = 1;
-  for (int n = 1; n <= 4; n++) {
+  for (int n = 1; n <= (every ? 4 : 3); n++) {
     const int gx = (tn + n - 1) / n;
     for (int rounds = 1; rounds <= 64; rounds++) {
       const int rb = rounds * 256 / gx;
       if (rb < 1) continue;
       int m = (tm + rb - 1) / rb;
-      if (bits == 4) m = m == 7 ? 8 : m;
+      if (every) m = m == 7 ? 8 : m;
       else m = m == 3 ? 4 : m;
-      if (m > (bits != 4 ? 4 : n == 4 ? 6 : 8)) continue;
+      if (m > (!every ? 4 : n == 4 ? 6 : 8)) continue;
       const int cost = rounds * (m + n + 2);
       if (cost < best) best = cost, *mt = m, *nt = n;
     }
@@ -229,6 +236,7 @@ void pick_tiles(int M, int N, int bits, int* mt, int* nt) {
 }
 
 }  // namespace
+}  // namespace strip
 
 // The DMAs move whole 64-k halves: 16 bytes at a time of a and of 4-bit rows, 4 of the others, and two scales at once.
 bool mnb_strip_takes(const MnbArgs& a) {
@@ -240,9 +248,9 @@ bool mnb_strip_takes(const MnbArgs& a) {
 hipError_t launch_mnb_strip(const MnbArgs& a, hipStream_t s) {
   if (a.M < 1 || !a.a || !a.y || !mnb_strip_takes(a)) return hipErrorInvalidValue;
   int mt = 0, nt = 0;
-  pick_tiles(a.M, a.N, a.bits, &mt, &nt);
+  strip::pick_tiles(a.M, a.N, strip::every_tile(a), &mt, &nt);
 #define HA_STRIP_CASE(B, G, S) \
-  if (a.bits == B && a.group == G && a.asym == S) return launch_fmt<B, G, S>(a, mt, nt, s);
+  if (a.bits == B && a.group == G && a.asym == S) return strip::launch_fmt<B, G, S>(a, mt, nt, s);
   HA_STRIP_CASE(4, 32, false) HA_STRIP_CASE(4, 32, true) HA_STRIP_CASE(4, 64, false) HA_STRIP_CASE(4, 64, true)
   HA_STRIP_CASE(3, 32, false) HA_STRIP_CASE(3, 32, true) HA_STRIP_CASE(3, 64, false) HA_STRIP_CASE(3, 64, true)
   HA_STRIP_CASE(2, 32, false) HA_STRIP_CASE(2, 32, true) HA_STRIP_CASE(2, 64, false) HA_STRIP_CASE(2, 64, true)

@@ -205,3 +205,5 @@ hipError_t launch_add_bias(void* y, const float* c, int L, int N, hipStream_t s)
 }
 
 }  // namespace ha
+
+#include "mnb_strip.h"  // (here and not with the GEMM: mnb.hip's m0 is only ever set for 16-byte DMAs)

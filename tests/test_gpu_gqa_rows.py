@@ -1,4 +1,4 @@
-"""Short full-attention calls (gqa_rows.hip) at the edges of their groups, tiles and pieces: every row equals, bit for bit,
+"""Short full-attention calls (gqa_rows.h) at the edges of their groups, tiles and pieces: every row equals, bit for bit,
 the same row of one long forward, which runs the general kernel; rows of both types; the caches a short call writes; a
 wait that runs out is reported."""
 import numpy as np
