@@ -550,8 +550,7 @@ def main():
                      "frac": round(achieved / 8000.0, 4), "traffic": measured_traffic(),
                      "bytes_per_launch": gdn_bytes, "bytes_per_token": gdn_bytes_per_token(),
                      "launch_ms": round(gdn_launch_ms, 5),
-                     "timing": "30 back-to-back one-layer forwards after 3 warm-up, HIP events on the launch stream; "
-                               "includes the layer's 3-row tail copy kernel (about 2% of it)"},
+                     "timing": "30 back-to-back one-layer forwards after 3 warm-up, HIP events on the launch stream"},
         "roofline_gqa": {"bound": "mfma", "kernel": "gqa_kv_kernel + gqa_attn_kernel",
                          "achieved": round(gqa_tf, 1), "peak": 2500.0, "unit": "TFLOP/s",
                          "frac": round(gqa_tf / 2500.0, 4), "flops_per_launch": B * gqa_flops(T),

@@ -97,7 +97,7 @@ typedef struct ha_forward_opts {
   int sync;        /* 1: wait for the stream before returning */
   float gpu_ms;    /* out: forward time when timestamps = 1 (implies a wait) */
   float* layer_ms; /* optional out [n_layers]: per-layer GPU ms (the reference's profile(), engine.js:292-307),
-                      each gated-delta layer's raw-row tail copy included */
+                      each gated-delta layer's raw-row tail copy included where a snapshot is kept */
   float* mixer_ms; /* optional out [n_layers]: GPU ms of each layer's token-mixer kernels alone (without the tail
                       copy; 0 for adapter layers). No counterpart in the reference: the kernel time a roofline is
                       computed on. Implies a wait, like layer_ms */

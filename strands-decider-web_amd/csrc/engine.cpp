@@ -1,7 +1,7 @@
 // Host side of the MI355X hybrid-attention engine: the C ABI declared in include/ha.h.
 //
 // Mirrors the reference engine's host logic for the token mixers (web/public/engine/engine.js):
-//   constructor buffers (engine.js:89-107)        -> ha_create: per-layer state, raw-row tail, K/V cache, RoPE table
+//   constructor buffers (engine.js:89-107)        -> ha_create: per-layer state, K/V cache, RoPE table
 //   plan() linear / full branches (253-276)       -> ha_forward: layer-kind dispatch, one stream, layers in order
 //   forward() resume (325-328)                    -> the snapshot's state / tail feed the kernels; K/V rows copied
 //   forward() snapshot (349-362)                  -> ha_forward(keep): new device buffers sized to the context
@@ -45,7 +45,6 @@ int fail(int code, const std::string& msg) {
 
 constexpr uint32_t kEngineMagic = 0x4841454eu, kSnapMagic = 0x48415350u, kDeadMagic = 0xdeadbeefu;
 constexpr int kKC = 4;                          // conv kernel the kernels are built for
-constexpr int kTailCap = ha::kChunk - 1 + kKC;  // at most 63 open rows + 3 history rows (+1 spare)
 std::atomic<uint64_t> g_engine_ids{1};
 std::atomic<uint64_t> g_snap_uid{0};  // snapshot uids: 1, 2, ...
 // Engines that exist right now. Handle checks look a pointer up here before reading through it, so a snapshot
@@ -67,8 +66,7 @@ struct Layer {
   float* gnorm = nullptr;
   float* qn = nullptr;
   float* kn = nullptr;
-  float* S = nullptr;     // [B][H][DK][DV] working state
-  void* tail = nullptr;   // [B][kTailCap][lin_stride] working raw-row tail
+  float* S = nullptr;     // [B][H][DK][DV] state of a call that keeps no snapshot
   _Float16* K = nullptr;  // [B][HK][LT][HD]
   _Float16* V = nullptr;  // [B][HK][HD][LT] (transposed: positions contiguous)
 };
@@ -251,7 +249,7 @@ void free_engine(ha_engine* e) {
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   for (auto& l : e->layers) {
     for (void* p : {(void*)l.conv, (void*)l.negA, (void*)l.dtb, (void*)l.gnorm, (void*)l.qn, (void*)l.kn, (void*)l.S,
-                    l.tail, (void*)l.K, (void*)l.V})
+                    (void*)l.K, (void*)l.V})
       if (p) (void)hipFree(p);
   }
   if (e->rope) (void)hipFree(e->rope);
@@ -297,6 +295,19 @@ void free_snapshot_buffers(ha_snapshot* s) {
   s->block = nullptr;
   s->block_bytes = 0;
 }
+
+// A snapshot under construction: given up, with its memory, unless the call completes.
+struct SnapshotGuard {
+  ha_snapshot* s;
+  hipStream_t st;
+  ~SnapshotGuard() {
+    if (!s) return;
+    (void)hipStreamSynchronize(st);  // queued kernels may write into its block
+    free_snapshot_buffers(s);
+    s->magic = kDeadMagic;
+    delete s;
+  }
+};
 
 // A bounded cross-workgroup wait of one of e's launches ran out (see ha::WaitCheck): report it once, as
 // HA_ERR_DEVICE, and clear the word. The engine.js counterpart throws the device errors a forward collected
@@ -404,14 +415,12 @@ int ha_create(const ha_config* cfg, int device, ha_engine** out) {
     if (l.kind == HA_LINEAR_ATTENTION) {
       e->any_linear = true;
       e->C = 2 * c.H * c.DK + c.H * c.DV;
-      const size_t esz = dtype_size(c.lin_dtype);
       if ((rc = dalloc(&l.conv, sizeof(float) * e->C * kKC)) || (rc = dalloc(&l.negA, sizeof(float) * c.H)) ||
           (rc = dalloc(&l.dtb, sizeof(float) * c.H)) || (rc = dalloc(&l.gnorm, sizeof(float) * c.DV)) ||
-          (rc = dalloc(&l.S, sizeof(float) * B * c.H * c.DK * c.DV)) ||
-          (rc = dalloc(&l.tail, esz * B * kTailCap * c.lin_stride)))
+          (rc = dalloc(&l.S, sizeof(float) * B * c.H * c.DK * c.DV)))
         return bail(rc);
       if (hipMemset(l.conv, 0, sizeof(float) * e->C * kKC) != hipSuccess || hipMemset(l.negA, 0, sizeof(float) * c.H) != hipSuccess ||
-          hipMemset(l.dtb, 0, sizeof(float) * c.H) != hipSuccess || hipMemset(l.tail, 0, esz * B * kTailCap * c.lin_stride) != hipSuccess)
+          hipMemset(l.dtb, 0, sizeof(float) * c.H) != hipSuccess)
         return bail(fail(HA_ERR_DEVICE, "hipMemset failed"));
       if ((rc = fill_f32(l.gnorm, c.DV, 1.0f))) return bail(rc);
     } else if (l.kind == HA_FULL_ATTENTION) {
@@ -663,13 +672,55 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
     int rc;  // first call that forces the paired form on another shape
     if ((rc = grow(sc.duo_ring, e->need_duo_ring))) return rc;
   }
-  // raw-row tails: the copy reads only the call's input rows and the resumed tail, so the layers' copies are
-  // gathered into one launch after the mixers (per layer when per-layer times are asked for, so that each layer's
-  // time includes its own copy)
+  // the snapshot's memory first: the gated-delta layers write their state and raw rows straight into it. Every part is in
+  // one device block (256-byte aligned offsets), the engine's spare block when it is large enough; a new block is rounded up
+  // to 2 MiB so that the next snapshots of a growing context fit in it when it returns
+  SnapshotGuard kept{nullptr, st};
+  if (keep) {
+    ha_snapshot* s = kept.s = new ha_snapshot();
+    s->owner = e; s->owner_id = e->id; s->uid = ++g_snap_uid; s->P = end; s->s0 = e->any_linear ? s1 : end;
+    s->tail_rows = s->P - (s->s0 - (kKC - 1));
+    s->layers.resize(c.n_layers);
+    auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t state = sizeof(float) * B * c.H * c.DK * c.DV, tail = dtype_size(c.lin_dtype) * c.lin_stride * B * s->tail_rows;
+    const size_t kv = (size_t)end * c.HD * sizeof(_Float16) * B * c.HK;
+    size_t total = 0;
+    for (const Layer& l : e->layers)
+      total += l.kind == HA_LINEAR_ATTENTION ? al(state) + al(tail) : l.kind == HA_FULL_ATTENTION ? 2 * al(kv) : 0;
+    {
+      std::lock_guard<std::mutex> lock(g_live_mu);
+      if (e->spare && e->spare_bytes >= total) {
+        s->block = e->spare; s->block_bytes = e->spare_bytes;
+        e->spare = nullptr; e->spare_bytes = 0;
+      }
+    }
+    if (!s->block) {
+      const size_t bytes = (total + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+      int rc = dalloc(reinterpret_cast<char**>(&s->block), bytes);
+      if (rc) return rc;
+      s->block_bytes = bytes;
+    }
+    size_t off = 0;
+    auto take = [&](size_t b) { void* q = static_cast<char*>(s->block) + off; off += al(b); return q; };
+    for (int i = 0; i < c.n_layers; i++) {
+      ha_snapshot::Part& p = s->layers[i];
+      if (e->layers[i].kind == HA_LINEAR_ATTENTION) {
+        p.S = static_cast<float*>(take(state));
+        p.tail = take(tail);
+      } else if (e->layers[i].kind == HA_FULL_ATTENTION) {
+        p.K = static_cast<_Float16*>(take(kv));
+        p.V = static_cast<_Float16*>(take(kv));
+      }
+    }
+  }
+  // raw-row tails of a kept snapshot: the copy reads only the call's input rows and the resumed tail, so the layers'
+  // copies are gathered into one launch after the mixers (per layer when per-layer times are asked for, so that each
+  // layer's time includes its own copy). A call that keeps no snapshot copies nothing: only a snapshot's rows are read
+  // again (4 - 5 us a call measured)
   ha::TailArgs t{};
   t.B = c.batch; t.stride = c.lin_stride; t.C = e->C; t.ab_off = e->C + c.H * c.DV; t.ab_n = 2 * c.H;
   t.P = P; t.L = L; t.s0 = s0; t.KC = kKC; t.tail_cap_in = resume ? resume->tail_rows : kKC - 1;
-  t.tail_cap_out = kTailCap; t.dst_first = s1 - (kKC - 1); t.dtype = c.lin_dtype == HA_F16 ? 1 : 0;
+  t.tail_cap_out = keep ? kept.s->tail_rows : 0; t.dst_first = s1 - (kKC - 1); t.dtype = c.lin_dtype == HA_F16 ? 1 : 0;
   auto flush_tails = [&]() {
     const hipError_t he = ha::launch_tail_update(t, st);
     t.n = 0;
@@ -687,7 +738,8 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       a.tail_cap = resume ? resume->tail_rows : kKC - 1;
       a.dtype = c.lin_dtype == HA_F16 ? 1 : 0;
       a.in = layer_in[i]; a.out = layer_out[i];
-      a.S_in = resume ? resume->layers[i].S : nullptr; a.S_out = l.S;
+      a.S_in = resume ? resume->layers[i].S : nullptr; a.S_out = keep ? kept.s->layers[i].S : l.S;
+      a.keep_state = keep != nullptr;
       a.conv_w = l.conv; a.negA = l.negA; a.dtb = l.dtb; a.gnorm = c.lin_gnorm ? l.gnorm : nullptr;
       a.img = sc.img.p; a.img_chunks = e->img_chunks;
       a.seq_raw = static_cast<float*>(sc.seq_raw.p); a.seq_cnt = static_cast<unsigned*>(sc.seq_cnt.p);
@@ -712,8 +764,10 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       }
       if (he != hipSuccess) return fail(HA_ERR_DEVICE, "layer " + std::to_string(i) + " gated-delta launch: " + hipGetErrorString(he));
       if (per_layer) HA_HIP(hipEventRecord(e->mev[i], st));
-      t.in[t.n] = a.in; t.tail[t.n] = a.tail; t.tail_out[t.n] = l.tail; t.n++;
-      if (per_layer || t.n == ha::kTailLayers) {
+      if (keep) {
+        t.in[t.n] = a.in; t.tail[t.n] = a.tail; t.tail_out[t.n] = kept.s->layers[i].tail; t.n++;
+      }
+      if (t.n > 0 && (per_layer || t.n == ha::kTailLayers)) {
         he = flush_tails();
         if (he != hipSuccess) return fail(HA_ERR_DEVICE, "layer " + std::to_string(i) + " tail update: " + hipGetErrorString(he));
       }
@@ -754,63 +808,22 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
   if (timing) HA_HIP(hipEventRecord(e->ev[1], st));
 
   if (keep) {
-    ha_snapshot* s = new ha_snapshot();
-    s->owner = e; s->owner_id = e->id; s->uid = ++g_snap_uid; s->P = end; s->s0 = e->any_linear ? s1 : end;
-    s->tail_rows = s->P - (s->s0 - (kKC - 1));
-    s->layers.resize(c.n_layers);
-    auto bail = [&](int code) { (void)hipStreamSynchronize(st); free_snapshot_buffers(s); s->magic = kDeadMagic; delete s; return code; };
-    // every part in one device block (256-byte aligned offsets), the engine's spare block when it is large enough;
-    // a new block is rounded up to 2 MiB so that the next snapshots of a growing context fit in it when it returns
-    auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    size_t total = 0;
-    for (int i = 0; i < c.n_layers; i++) {
-      const Layer& l = e->layers[i];
-      if (l.kind == HA_LINEAR_ATTENTION)
-        total += al(sizeof(float) * B * c.H * c.DK * c.DV) + al(dtype_size(c.lin_dtype) * c.lin_stride * B * s->tail_rows);
-      else if (l.kind == HA_FULL_ATTENTION)
-        total += 2 * al((size_t)end * c.HD * sizeof(_Float16) * B * c.HK);
-    }
-    {
-      std::lock_guard<std::mutex> lock(g_live_mu);
-      if (e->spare && e->spare_bytes >= total) {
-        s->block = e->spare; s->block_bytes = e->spare_bytes;
-        e->spare = nullptr; e->spare_bytes = 0;
-      }
-    }
-    if (!s->block) {
-      const size_t bytes = (total + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
-      int rc = dalloc(reinterpret_cast<char**>(&s->block), bytes);
-      if (rc) return bail(rc);
-      s->block_bytes = bytes;
-    }
-    size_t off = 0;
-    auto take = [&](size_t b) { void* q = static_cast<char*>(s->block) + off; off += al(b); return q; };
+    ha_snapshot* s = kept.s;
     for (int i = 0; i < c.n_layers; i++) {
       Layer& l = e->layers[i];
       ha_snapshot::Part& p = s->layers[i];
-      if (l.kind == HA_LINEAR_ATTENTION) {
-        const size_t sb = sizeof(float) * B * c.H * c.DK * c.DV, esz = dtype_size(c.lin_dtype);
-        const size_t rowb = esz * c.lin_stride;
-        p.S = static_cast<float*>(take(sb));
-        p.tail = take(rowb * B * s->tail_rows);
-        if (hipMemcpyAsync(p.S, l.S, sb, hipMemcpyDeviceToDevice, st) != hipSuccess ||
-            hipMemcpy2DAsync(p.tail, rowb * s->tail_rows, l.tail, rowb * kTailCap, rowb * s->tail_rows, B,
-                             hipMemcpyDeviceToDevice, st) != hipSuccess)
-          return bail(fail(HA_ERR_DEVICE, "snapshot copy failed"));
-      } else if (l.kind == HA_FULL_ATTENTION) {
-        const size_t w = (size_t)end * c.HD * sizeof(_Float16), sp = (size_t)c.max_ctx * c.HD * sizeof(_Float16);
-        const size_t vw = (size_t)end * sizeof(_Float16), vp = (size_t)c.max_ctx * sizeof(_Float16);
-        p.K = static_cast<_Float16*>(take(w * B * c.HK));
-        p.V = static_cast<_Float16*>(take(w * B * c.HK));
-        if (hipMemcpy2DAsync(p.K, w, l.K, sp, w, B * c.HK, hipMemcpyDeviceToDevice, st) != hipSuccess ||
-            hipMemcpy2DAsync(p.V, vw, l.V, vp, vw, B * c.HK * c.HD, hipMemcpyDeviceToDevice, st) != hipSuccess)
-          return bail(fail(HA_ERR_DEVICE, "snapshot copy failed"));
-      }
+      if (l.kind != HA_FULL_ATTENTION) continue;
+      const size_t w = (size_t)end * c.HD * sizeof(_Float16), sp = (size_t)c.max_ctx * c.HD * sizeof(_Float16);
+      const size_t vw = (size_t)end * sizeof(_Float16), vp = (size_t)c.max_ctx * sizeof(_Float16);
+      if (hipMemcpy2DAsync(p.K, w, l.K, sp, w, B * c.HK, hipMemcpyDeviceToDevice, st) != hipSuccess ||
+          hipMemcpy2DAsync(p.V, vw, l.V, vp, vw, B * c.HK * c.HD, hipMemcpyDeviceToDevice, st) != hipSuccess)
+        return fail(HA_ERR_DEVICE, "snapshot copy failed");
     }
     {
       std::lock_guard<std::mutex> lock(g_live_mu);
       g_live_snaps.insert(s);
     }
+    kept.s = nullptr;
     *keep = s;
   }
   if (timing || (opts && opts->sync)) {
@@ -889,7 +902,7 @@ int ha_snapshot_read(const ha_snapshot* s, int layer, const char* what, void* ho
     a.P = s->P; a.L = 0; a.s0 = s->s0;
     a.tail = s->layers[layer].tail; a.tail_cap = s->tail_rows;
     a.dtype = c.lin_dtype == HA_F16 ? 1 : 0;
-    a.S_in = s->layers[layer].S; a.S_out = tmp;
+    a.S_in = s->layers[layer].S; a.S_out = tmp; a.keep_state = true;
     a.conv_w = l.conv; a.negA = l.negA; a.dtb = l.dtb; a.gnorm = nullptr;  // no output rows: replay only
     hipError_t he = ha::launch_gdn_sequential(a, e->stream);
     if (he == hipSuccess) he = hipMemcpyAsync(host, tmp, want, hipMemcpyDeviceToHost, e->stream);

@@ -38,7 +38,8 @@ struct GdnArgs {
   const void* tail;                 // [B][tail_cap][stride]
   void* out;                        // [B][L][H*DV]
   const float* S_in;                // [B][H][DK][DV] state at s0, or nullptr for a zero state
-  float* S_out;                     // [B][H][DK][DV] state at the returned position (may equal S_in)
+  float* S_out;                     // [B][H][DK][DV] state at the returned position
+  bool keep_state;                  // the caller reads S_out afterwards (the sequential form leaves it unwritten otherwise)
   const float* conv_w;              // [C][KC]
   const float* negA;                // [H]
   const float* dtb;                 // [H]
@@ -104,7 +105,7 @@ struct TailArgs {
   int n;                          // layers in this launch, 1..kTailLayers
   const void* in[kTailLayers];    // per layer: the call's input rows, [B][L][stride]
   const void* tail[kTailLayers];  // per layer: the raw-row tail the call resumed from, [B][tail_cap_in][stride]
-  void* tail_out[kTailLayers];    // per layer: the working raw-row tail, [B][tail_cap_out][stride]
+  void* tail_out[kTailLayers];    // per layer: the snapshot's raw-row tail, [B][tail_cap_out][stride]
 };
 
 hipError_t launch_gdn_sequential(const GdnArgs& a, hipStream_t s);
