@@ -1043,13 +1043,12 @@ int mnb_forward(ha_mnb* w, int M, const void* a, void* y, void* stream, bool noa
   hipStream_t st = (hipStream_t)stream;
   ha::MnbArgs g = w->args;
   g.M = M; g.a = a; g.y = y;
-  if (ha::mnb_strip_path(g)) {
-    HA_HIP(ha::launch_mnb_strip(g, st));
-    return HA_OK;
-  }
-  if (ha::mnb_packed_path(M, g.N, g.K)) {
-    HA_HIP(ha::launch_mnb_gemv(g, st));
-    return HA_OK;
+  g.ldy = g.N;
+  switch (ha::mnb_path(g)) {
+    case ha::kMnbGemv: HA_HIP(ha::launch_mnb_gemv(g, st)); return HA_OK;
+    case ha::kMnbStrip: HA_HIP(ha::launch_mnb_strip(g, st)); return HA_OK;
+    case ha::kMnbTiles: HA_HIP(ha::launch_mnb_tiles(g, st)); return HA_OK;
+    case ha::kMnbGemm: break;
   }
   g.split = ha::mnb_gemm_split(M, g.N, g.K);
   if (g.split > 1 && noalloc) {

@@ -126,15 +126,20 @@ struct MnbArgs {
   const void* q;  // [N][K/32][bits] u32
   const void* s;  // [N][K/group] f16
   const void* b;  // [N][K/group] f16 (asymmetric only)
+  int ldy = 0;          // elements between rows of y (the strip and tile kernels; N)
   int split = 1;     // GEMM only: K ranges, each on its own workgroups, summed in order by a second kernel
   float* ws = nullptr;  // [split][M][N] fp32 partial products when split > 1
 };
 hipError_t mnb_check(const MnbArgs& a);
-bool mnb_packed_path(int M, int N, int K);  // whether launch_mnb_gemv (packed weights) serves M rows
 bool mnb_strip_takes(const MnbArgs& a);     // whether launch_mnb_strip can run these operands (K, alignment)
-bool mnb_strip_path(const MnbArgs& a);      // whether it serves them
+float mnb_strip_us(const MnbArgs& a);       // the time it is expected to take
 hipError_t launch_mnb_strip(const MnbArgs& a, hipStream_t s);
-hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s);  // M <= 64 (mnb_packed_path picks up to 48)
+bool mnb_tiles_takes(const MnbArgs& a);     // likewise launch_mnb_tiles (4-bit weights)
+float mnb_tiles_us(const MnbArgs& a);
+hipError_t launch_mnb_tiles(const MnbArgs& a, hipStream_t s);
+enum MnbPath { kMnbGemv, kMnbStrip, kMnbTiles, kMnbGemm };
+MnbPath mnb_path(const MnbArgs& a);         // the kernel that serves a call
+hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s);  // M <= 64
 int mnb_gemm_split(int M, int N, int K);  // K ranges the GEMM uses for this shape (1: none, no workspace)
 hipError_t launch_mnb_gemm(const MnbArgs& a, hipStream_t s);  // any M: tiled GEMM, weights dequantised into LDS
 // Scratch of the allocation-free GEMM entry point (mnb.hip): a file-scope device array of kMnbScratchBytes per GPU.

@@ -10,17 +10,19 @@
 //   hold the low two bits as in the 2-bit layout and bit e of word 2 is element e's high bit. One f16 scale per
 //   `group` (32 or 64) values of a row; symmetric w = (q - 2^(bits-1)) * scale, asymmetric w = q * scale + bias.
 //
-// Implementations, chosen by M as the reference chooses its kernels by M:
+// Implementations, chosen by M as the reference chooses its kernels by M (mnb_path):
 //   M <= 2    mnb_gemv_lanes_kernel: weight-bandwidth bound. A wave owns 4 output columns, its lanes run along K
 //             over whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
-//   M <= 384  mnb_strip_kernel (mnb_strip.h): each wave of a workgroup takes a part of K through LDS of its own.
-//   M <= 64   mnb_gemv_kernel, where the operands do not suit the strip kernel's DMAs (mnb_strip_takes): a workgroup
-//             owns 16 output columns and its 8 waves split the K blocks; each lane dequantises a whole packed block
-//             into the f16 B operands of v_mfma_f32_16x16x32_f16 (no LDS), the a rows are the A operand (16 rows per
-//             tile, up to 4 tiles share each dequantised operand), and the waves' partial sums meet in LDS.
-//   above     mnb_gemm_kernel: compute bound. A tiled MFMA GEMM (128 or 256 x 128 workgroup tiles) whose weight
-//             tiles are dequantised on their way into LDS, so the weights stay packed in HBM. With few output tiles
-//             the K range is split over workgroups and mnb_split_sum_kernel adds the fp32 partials in order.
+//   few rows  mnb_strip_kernel (mnb_strip.h): each wave of a workgroup takes a part of K through LDS of its own.
+//   many rows mnb_tiles_kernel (mnb_tiles.h, 4 bits): MFMA tiles, weights dequantised in registers.
+// and for operands that do not suit the DMAs of those two (K % 64, alignment), or 2 and 3 bits above 384 rows:
+//   M <= 64   mnb_gemv_kernel: a workgroup owns 16 output columns and its 8 waves split the K blocks; each lane
+//             dequantises a whole packed block into the f16 B operands of v_mfma_f32_16x16x32_f16 (no LDS), the a rows
+//             are the A operand (16 rows per tile, up to 4 tiles share each dequantised operand), and the waves'
+//             partial sums meet in LDS.
+//   above     mnb_gemm_kernel: a tiled MFMA GEMM (128 or 256 x 128 workgroup tiles) whose weight tiles are dequantised
+//             on their way into LDS. With few output tiles the K range is split over workgroups and
+//             mnb_split_sum_kernel adds the fp32 partials in order.
 // All dequantise with the same f16 arithmetic (each weight rounded to f16 once), accumulate in
 // fp32 and round the output to f16. Results are deterministic: a split K range is summed in a fixed order that
 // depends only on the shape.
@@ -498,17 +500,15 @@ hipError_t mnb_check(const MnbArgs& a) {
   return hipSuccess;
 }
 
-bool mnb_packed_path(int M, int N, int K) {
-  // Measured on MI355X, back-to-back calls on the model's projection shapes (N x K from 2048 x 2048 to
-  // 12288 x 2048): up to 64 rows the packed-weight kernels are at least as fast as the tiled GEMM on every shape
-  // (at 64 rows 10-28 us against 27-71 us).
-  return M <= 64;
-}
-
-bool mnb_strip_path(const MnbArgs& a) {
-  // Up to 384 rows the strip kernel is faster than the tiled GEMM on every projection shape (333 rows: 8 - 35 us against
-  // 20 - 43 us); at 512 rows the GEMM wins on 12288 x 2048 (45 against 49 us). One or two rows: the lanes kernel.
-  return a.M > kLanesRows && a.M <= 384 && mnb_strip_takes(a);
+MnbPath mnb_path(const MnbArgs& a) {
+  // One or two rows: the lanes kernel. Operands that the DMAs of the strip and tile kernels cannot move (K % 64, alignment):
+  // the register-operand kernel up to 64 rows (10 - 28 us at 64 rows against 27 - 71 us for the GEMM), then the GEMM.
+  if (a.M <= kLanesRows) return kMnbGemv;
+  if (!mnb_strip_takes(a)) return a.M <= 64 ? kMnbGemv : kMnbGemm;
+  if (!mnb_tiles_takes(a)) return a.M <= 384 ? kMnbStrip : kMnbGemm;  // 2 and 3 bits
+  // 4 bits: up to 256 rows the strip kernel (a row's bits then depend on neither M nor the tiles), above it the one whose
+  // expected time is less
+  return a.M <= 256 || mnb_strip_us(a) < mnb_tiles_us(a) ? kMnbStrip : kMnbTiles;
 }
 
 hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s) {
@@ -571,3 +571,5 @@ hipError_t launch_fwht(void* x, long rows_times_k, int n, hipStream_t s) {
 }
 
 }  // namespace ha
+
+#include "mnb_tiles.h"

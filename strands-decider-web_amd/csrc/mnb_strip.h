@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64 * kSW) void mnb_strip_kernel(MnbArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int m = m0 + 16 * (q / NT) + 4 * g + e;
-      if (m < a.M && n < a.N) ((_Float16*)a.y)[(size_t)m * a.N + n] = (_Float16)s[e];
+      if (m < a.M && n < a.N) ((_Float16*)a.y)[(size_t)m * a.ldy + n] = (_Float16)s[e];
     }
   }
 }
@@ -216,7 +216,7 @@ hipError_t launch_fmt(const MnbArgs& a, int mt, int nt, hipStream_t s) {
 // workgroups a round, over the rounds that needs, and of those the least rounds x (mt + nt + 2). Measured choices
 // (M, N, K: mt x nt us, next best): 61, 2048, 6144: 2 x 1 8.0, 3 x 1 9.0; 61, 12288, 2048: 4 x 3 9.9, 2 x 3 10.4;
 // 128, 5120, 2048: 3 x 4 8.9, 4 x 3 9.1; 192, 8256, 2048: 4 x 4 18.0, 3 x 3 18.7.
-void pick_tiles(int M, int N, bool every, int* mt, int* nt) {
+int pick_tiles(int M, int N, bool every, int* mt, int* nt) {
   const int tm = (M + 15) / 16, tn = N / 16;
   int best = 1 << 30;
   *mt = *nt = 1;
@@ -233,6 +233,7 @@ void pick_tiles(int M, int N, bool every, int* mt, int* nt) {
       if (cost < best) best = cost, *mt = m, *nt = n;
     }
   }
+  return best;
 }
 
 }  // namespace
@@ -243,6 +244,12 @@ bool mnb_strip_takes(const MnbArgs& a) {
   const uintptr_t q = (uintptr_t)a.q, sb = (uintptr_t)a.s | (a.asym ? (uintptr_t)a.b : 0);
   return a.K % 64 == 0 && (a.group == 32 || a.K % 128 == 0) && (uintptr_t)a.a % 16 == 0 &&
          q % (a.bits == 4 ? 16 : 4) == 0 && sb % 4 == 0;
+}
+
+// rounds x (mt + nt + 2), in units of 0.35 us and 0.55 us for every 2048 of K (measured 0.8 to 1.1 of this)
+float mnb_strip_us(const MnbArgs& a) {
+  int mt, nt;
+  return (float)strip::pick_tiles(a.M, a.N, strip::every_tile(a), &mt, &nt) * (0.35f + 0.55f * a.K / 2048.0f);
 }
 
 hipError_t launch_mnb_strip(const MnbArgs& a, hipStream_t s) {

@@ -1,4 +1,4 @@
-"""The strip kernel of the MatMulNBits projections (3 to 384 rows) at the edges of its tiles, against the fp64 oracle: one
+"""The strip kernel of the MatMulNBits projections (from 3 rows on) at the edges of its tiles, against the fp64 oracle: one
 and two rows around each count of 16-row tiles, a column count that no tile count divides, K of one half, an odd number
 of halves and more groups than waves, every weight format; rows that keep their bits whatever M is; operands whose
 alignment sends the call to the general kernels."""
@@ -44,7 +44,7 @@ def test_tile_edges(N, K, bits, group, asym):
     a = ((np.random.default_rng(1).random((385, K)) - 0.5) * 2).astype(np.float16)
     ad, ref = _dev(a), mo.matmul(a, W)
     full = None
-    for M in (384, 3, 15, 16, 17, 32, 33, 49, 65, 81, 97, 113, 129, 193, 257, 385):
+    for M in (256, 3, 15, 16, 17, 32, 33, 49, 65, 81, 97, 113, 129, 193, 257, 384, 385):
         y = torch.full((M + 1, N), 7.0, dtype=torch.float16, device="cuda:0")
         w.forward(M, ad, y)
         torch.cuda.synchronize()
@@ -53,8 +53,33 @@ def test_tile_edges(N, K, bits, group, asym):
         assert (g[M] == 7.0).all(), "row past M written (M = %d)" % M
         if full is None:
             full = g
-        elif M < 384 and K % 64 == 0 and (group == 32 or K % 128 == 0):
+        elif M < 256 and K % 64 == 0 and (group == 32 or K % 128 == 0):
             assert np.array_equal(g[:M].view(np.uint16), full[:M].view(np.uint16)), "bits of a row depend on M = %d" % M
+    w.close()
+
+
+@pytest.mark.parametrize("N,K,group,asym", [
+    (4160, 192, 32, False), (4112, 448, 32, True), (3008, 1024, 64, False), (8256, 128, 64, True), (5120, 64, 32, False)])
+def test_many_rows(N, K, group, asym):
+    # more rows than the strip kernel is the faster for: the tile kernel, at edges of its tiles in both directions (a last
+    # column tile of 16, 64, 192 and 256; rows just over and under a multiple of 128 and 256) and of its six-tile K loop;
+    # rows keep their bits whatever M is
+    import torch
+    words, sc, bi = _weights(N, K, 4, group, asym, N + K)
+    W = mo.dequant(words, sc, N, K, 4, group, asym, bi)
+    q, s, b = _dev(words), _dev(sc), _dev(bi) if asym else None
+    w = ha.MnbWeight(N, K, q, s, b, bits=4, group=group, asym=asym)
+    a = ((np.random.default_rng(3).random((2050, K)) - 0.5) * 2).astype(np.float16)
+    ad, ref, full = _dev(a), mo.matmul(a, W), None
+    for M in (2050, 1025, 1151, 1409):
+        y = torch.full((M + 1, N), 7.0, dtype=torch.float16, device="cuda:0")
+        w.forward(M, ad, y)
+        torch.cuda.synchronize()
+        g = y.cpu().numpy()
+        assert mo.rel_err(g[:M].astype(np.float64), ref[:M]) < TOL, M
+        assert (g[M] == 7.0).all(), "row past M written (M = %d)" % M
+        full = g if full is None else full
+        assert np.array_equal(g[:M].view(np.uint16), full[:M].view(np.uint16)), "bits of a row depend on M = %d" % M
     w.close()
 
 
