@@ -11,8 +11,8 @@
 //   `group` (32 or 64) values of a row; symmetric w = (q - 2^(bits-1)) * scale, asymmetric w = q * scale + bias.
 //
 // Implementations, chosen by M as the reference chooses its kernels by M (mnb_path):
-//   M <= 2    mnb_gemv_lanes_kernel: weight-bandwidth bound. A wave owns 4 output columns, its lanes run along K
-//             over whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
+//   M <= 2    mnb_gemv_lanes_kernel (below 4096 columns): a wave owns 2 output columns, its lanes run along K over
+//             whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
 //   few rows  mnb_strip_kernel (mnb_strip.h): each wave of a workgroup takes a part of K through LDS of its own.
 //   many rows mnb_tiles_kernel (mnb_tiles.h, 4 bits): MFMA tiles, weights dequantised in registers.
 // and for operands that do not suit the DMAs of those two (K % 64, alignment), or 2 and 3 bits above 384 rows:
@@ -163,45 +163,76 @@ __global__ __launch_bounds__(64 * kGW) void mnb_gemv_kernel(MnbArgs a) {
   }
 }
 
-// y for M = MR <= 2 rows: a wave owns kLW consecutive output columns and its lanes run along K. Lane l takes
-// blocks l, l + 64, ... of each of its columns (one whole-block load per column, so a wave instruction reads a
-// contiguous 1 KiB of one column's packed row), dequantises them to f16 pairs and multiplies them into the rows of a
-// with v_dot2_f32_f16 (fp32 accumulation); the a values are loaded once per block for all the columns. The lanes'
-// partial sums are reduced across the wave. Grid: N / (4 kLW) workgroups of 4 waves.
-constexpr int kLW = 4;
-template <int BITS, int GROUP, bool ASYM, int MR>
+// y for M = MR <= 2 rows: a wave owns LW consecutive output columns and its lanes run along K. Lane l takes blocks l,
+// l + 64, ... of each of its columns (one whole-block load per column, so a wave instruction reads a contiguous 1 KiB of
+// one column's packed row), dequantises them and multiplies them into the rows of a with v_dot2_f32_f16 (fp32
+// accumulation); the next blocks are loaded before the current ones are used. The lanes' partial sums are added by DPP and
+// permlane. Bound: round trips, in a kernel of a few us. With two columns a wave the rows of a come through LDS, copied once
+// per workgroup in whole lines while the first blocks are on their way: read directly, a lane's 64 bytes are a cache line
+// of their own, twice the address cycles of two columns' weights. With four the copy and its barrier cost more than it
+// saves. Grid: N / (4 LW) workgroups of 4 waves. 2048 x 6144: 6.1 -> 5.1 us with one row, 7.4 -> 5.6 with two (LW = 4 -> 2).
+constexpr int kLaneChunk = 8192;  // k of a in LDS at a time
+__device__ __forceinline__ float lanes_sum(float v) {
+  auto ror = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  v += ror(v, std::integral_constant<int, 0x128>{});  // row_ror:8, 4, 2, 1
+  v += ror(v, std::integral_constant<int, 0x124>{});
+  v += ror(v, std::integral_constant<int, 0x122>{});
+  v += ror(v, std::integral_constant<int, 0x121>{});
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  const unsigned t = __builtin_bit_cast(unsigned, v);
+  const auto q = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+  return __builtin_bit_cast(float, (unsigned)q[0]) + __builtin_bit_cast(float, (unsigned)q[1]);
+}
+template <int BITS, int GROUP, bool ASYM, int MR, int LW>
 __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
-  const int lane = threadIdx.x & 63, n0 = kLW * (4 * blockIdx.x + (threadIdx.x >> 6));
+  extern __shared__ __attribute__((aligned(16))) unsigned char al[];  // [row][16-byte chunks], chunk q at q ^ (q / 16 % 4)
+  const int tid = threadIdx.x, lane = tid & 63, n0 = LW * (4 * blockIdx.x + (tid >> 6));
   const int nblk = a.K / kBlk, ng = a.K / GROUP;
-  float acc[kLW][MR];
+  constexpr bool kStaged = LW == 2;
+  const int chunk = kStaged ? kLaneChunk : a.K;
+  struct Blk {
+    unsigned wd[LW][BITS];
+    unsigned short sc[LW], bi[LW];
+  };
+  auto load = [&](int b, Blk& x) {
+    b = min(b, nblk - 1);
 #pragma unroll
-  for (int c = 0; c < kLW; c++)
-#pragma unroll
-    for (int m = 0; m < MR; m++) acc[c][m] = 0.0f;
-  for (int b = lane; b < nblk; b += 64) {
-    unsigned wd[kLW][BITS];
-    h2 sc[kLW], bi[kLW];
-#pragma unroll
-    for (int c = 0; c < kLW; c++) {
+    for (int c = 0; c < LW; c++) {
       gptr<unsigned> wp = gp<unsigned>(a.q) + ((size_t)(n0 + c) * nblk + b) * BITS;
 #pragma unroll
-      for (int j = 0; j < BITS; j++) wd[c][j] = wp[j];
+      for (int j = 0; j < BITS; j++) x.wd[c][j] = wp[j];
       const size_t gi = (size_t)(n0 + c) * ng + b * kBlk / GROUP;
-      sc[c] = splat2(gp<_Float16>(a.s)[gi]);
-      bi[c] = splat2(ASYM ? gp<_Float16>(a.b)[gi] : (_Float16)0.0f);
+      x.sc[c] = gp<unsigned short>(a.s)[gi];
+      x.bi[c] = ASYM ? gp<unsigned short>(a.b)[gi] : 0;
     }
+  };
+  float acc[LW][MR];
+#pragma unroll
+  for (int c = 0; c < LW; c++)
+#pragma unroll
+    for (int m = 0; m < MR; m++) acc[c][m] = 0.0f;
+  auto use = [&](int b, int k0, const Blk& x) {
     h8 av[MR][4];
 #pragma unroll
-    for (int m = 0; m < MR; m++) {
-      gptr<h8> ap = (gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + (size_t)b * kBlk);
-#pragma unroll
-      for (int j = 0; j < 4; j++) av[m][j] = perm8(ap[j]);
-    }
-#pragma unroll
-    for (int c = 0; c < kLW; c++) {
+    for (int m = 0; m < MR; m++)
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        const h8 wv = dequant8_pk<BITS, ASYM>(wd[c], j, sc[c], bi[c]);
+        const int q = 4 * (b - k0 / kBlk) + j;
+        if constexpr (!kStaged) av[m][j] = *(gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + (size_t)b * kBlk + 8 * j);
+        else av[m][j] = *reinterpret_cast<const h8*>(al + (size_t)m * 2 * min(a.K, kLaneChunk) + 16 * (q ^ ((q >> 4) & 3)));
+      }
+#pragma unroll
+    for (int c = 0; c < LW; c++) {
+      const h2 sc = splat2u(x.sc[c]), bi = splat2u(x.bi[c]);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        h8 wv;
+        if constexpr (BITS == 4) wv = dequant8_nat4<ASYM>(x.wd[c][j], sc, bi);
+        else wv = dequant8_nat<BITS, ASYM>((x.wd[c][j >> 1] >> (16 * (j & 1))) & 0xFFFFu, BITS == 3 ? (x.wd[c][BITS - 1] >> (8 * j)) & 0xFFu : 0u, sc, bi);
 #pragma unroll
         for (int m = 0; m < MR; m++)
 #pragma unroll
@@ -210,14 +241,32 @@ __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
                                                acc[c][m], false);
       }
     }
+  };
+  Blk cur;
+  load(lane, cur);
+  for (int k0 = 0; k0 < a.K; k0 += chunk) {
+    const int n = min(a.K - k0, chunk);
+    if constexpr (kStaged) {
+      if (k0) __syncthreads();  // the chunk before has been read
+#pragma unroll
+      for (int m = 0; m < MR; m++)
+        for (int q = tid; q < n / 8; q += 256)
+          *reinterpret_cast<h8*>(al + (size_t)m * 2 * min(a.K, kLaneChunk) + 16 * (q ^ ((q >> 4) & 3))) =
+              *(gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + k0 + 8 * q);
+      __syncthreads();
+    }
+    for (int b = k0 / kBlk + lane; b < (k0 + n) / kBlk; b += 64) {
+      Blk next;
+      load(b + 64, next);
+      use(b, k0, cur);
+      cur = next;
+    }
   }
 #pragma unroll
-  for (int c = 0; c < kLW; c++)
+  for (int c = 0; c < LW; c++)
 #pragma unroll
     for (int m = 0; m < MR; m++) {
-      float v = acc[c][m];
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+      const float v = lanes_sum(acc[c][m]);
       if (lane == 0 && m < a.M) ((_Float16*)a.y)[(size_t)m * a.N + n0 + c] = (_Float16)v;
     }
 }
@@ -497,11 +546,18 @@ void launch_fwht_log(_Float16* x, long blocks, float scale, hipStream_t s) {
   hipLaunchKernelGGL(fwht_kernel<LOG>, dim3((unsigned)((blocks + kPer - 1) / kPer)), dim3(kWG), 0, s, x, blocks, scale);
 }
 
+template <int BITS, int GROUP, bool ASYM, int MR>
+void launch_lanes(const MnbArgs& a, hipStream_t s) {
+  if (a.N < 4096)
+    hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, MR, 2>), dim3(a.N / 8), dim3(256),
+                       (size_t)MR * 2 * std::min(a.K, kLaneChunk), s, a);
+  else
+    hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, MR, 4>), dim3(a.N / 16), dim3(256), 0, s, a);
+}
 template <int BITS, int GROUP, bool ASYM>
 hipError_t launch_gemv_lanes(const MnbArgs& a, hipStream_t s) {
-  const dim3 grid(a.N / (4 * kLW)), block(256);
-  if (a.M == 1) hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, 1>), grid, block, 0, s, a);
-  else if (a.M == 2) hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, 2>), grid, block, 0, s, a);
+  if (a.M == 1) launch_lanes<BITS, GROUP, ASYM, 1>(a, s);
+  else if (a.M == 2) launch_lanes<BITS, GROUP, ASYM, 2>(a, s);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
@@ -568,9 +624,10 @@ hipError_t mnb_check(const MnbArgs& a) {
 }
 
 MnbPath mnb_path(const MnbArgs& a) {
-  // One or two rows: the lanes kernel. Operands that the DMAs of the strip and tile kernels cannot move (K % 64, alignment):
+  // One or two rows: the lanes kernel, from 4096 columns on the strip kernel (12288 / 8256 / 5120 x 2048: 5.9 / 5.3 / 4.7
+  // us against 6.8 / 6.0 / 5.0; 2048 x 2048 / 6144: 4.6 / 6.3 against 3.8 / 5.1). Operands that the DMAs of the strip and tile kernels cannot move (K % 64, alignment):
   // the register-operand kernel up to 64 rows (10 - 28 us at 64 rows against 27 - 71 us for the GEMM), then the GEMM.
-  if (a.M <= kLanesRows) return kMnbGemv;
+  if (a.M <= kLanesRows) return a.N >= 4096 && mnb_strip_takes(a) ? kMnbStrip : kMnbGemv;
   if (!mnb_strip_takes(a)) return a.M <= 64 ? kMnbGemv : kMnbGemm;
   if (!mnb_tiles_takes(a)) return a.M <= 384 ? kMnbStrip : kMnbGemm;  // 2 and 3 bits
   // 4 bits: up to 256 rows the strip kernel (a row's bits then depend on neither M nor the tiles), above it the one whose
