@@ -18,8 +18,8 @@
 // Bound: latency (a dependent chain of launches, loads and one cross-workgroup hand-off); the K/V cache is read once.
 // Waits: a workgroup waits only for workgroups of lower index in its grid. Each XCD takes its blocks in order, so the
 // lowest unfinished block is always resident and waits for finished ones: every wait ends, and each is bounded besides.
-// Measured, f16 rows, us a call, before -> now: 61 rows after 1531 (1 sequence) 61 -> 25; one row after 1536 (8 sequences)
-// 56 -> 28 (scores 15.8, values 12.3), after 3000 93 -> 47; 64 rows of an empty context 26 -> 20.
+// Measured, f16 rows, us a call, before -> now: 61 rows after 1531 (1 sequence) 61 -> 23; one row after 1536 (8 sequences)
+// 56 -> 28 (scores 15.8, values 12.3), after 3000 93 -> 47; 64 rows of an empty context 26 -> 17.
 #pragma once
 #include <algorithm>
 
@@ -81,14 +81,22 @@ struct QRow {
   h8 raw[sizeof(T) == 2 ? 16 : 1];
   gptr<T> src;
   gptr<float> rp;
+  template <bool kStaged>
   __device__ __forceinline__ void load(const GqaArgs& a, int b, int h, int q0, int half, int c32) {
     const int tc = min(q0 + c32, a.L - 1);
     src = gp<T>(a.in) + ((size_t)b * a.L + tc) * a.stride + (size_t)h * 2 * kHD + 8 * half;
-    if constexpr (sizeof(T) == 2) {
+    if constexpr (sizeof(T) == 2 && !kStaged) {
 #pragma unroll
       for (int ks = 0; ks < 16; ks++) raw[ks] = *(gptr<h8>)(src + 16 * ks);
     }
     rp = gp<float>(a.rope) + (size_t)(a.P + tc) * a.RD + 16 * half;
+  }
+  // the same from the group's staged rows of this head: row r at 512 r, 16-byte chunk j in slot j ^ r
+  __device__ __forceinline__ void take(const unsigned char* ql, int half, int c32) {
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int ks = 0; ks < 16; ks++) raw[ks] = *reinterpret_cast<const h8*>(ql + 512 * c32 + 16 * ((2 * ks + half) ^ c32));
+    }
   }
   __device__ __forceinline__ void load_rope() {
 #pragma unroll
@@ -194,8 +202,15 @@ struct Raw4<float> { f4 v; };
 __device__ __forceinline__ f4 wide(const Raw4<_Float16>& x) { return f4{(float)x.v[0], (float)x.v[1], (float)x.v[2], (float)x.v[3]}; }
 __device__ __forceinline__ f4 wide(const Raw4<float>& x) { return x.v; }
 
-// 128 VGPRs: two workgroups a CU, so that a batch's tiles all run at once
-template <typename T>
+// 128 VGPRs: two workgroups a CU, so that a batch's tiles all run at once. kStaged (f16 rows, more than kDirect rows): the
+// group's q rows of the four heads come through LDS, copied once in whole lines; read directly, a lane's 16 bytes are a
+// cache line of their own, for both waves of a head (8K address cycles a workgroup against 1K). 64 KiB more LDS leaves one
+// workgroup a CU, so only in launches of at most one for each: 64 rows after 1531, B = 1 (104 workgroups) 25.4 -> 22.8 us
+// for both launches, after 500 24.4 -> 21.1; but 9 rows after 1531, B = 8 (400) 30 -> 34. Up to kDirect rows the lanes of a
+// direct load share lines: no gain.
+constexpr int kDirect = 8;
+constexpr int kQLds = 4 * 32 * 512;
+template <typename T, bool kStaged>
 __global__ __launch_bounds__(64 * kSW, 4) void gqa_scores_kernel(GqaArgs a) {
   // K tile as gqa_attn_kernel stages it: key r at [r][32 chunks of 8 dims], chunk j in slot j ^ (r & 31)
   // then, once S is made, the maxima of earlier halves
@@ -203,6 +218,7 @@ __global__ __launch_bounds__(64 * kSW, 4) void gqa_scores_kernel(GqaArgs a) {
   __shared__ __attribute__((aligned(16))) float qw_l[kHD];
   __shared__ f4 rope_l[kBK][16];  // the RoPE rows of the tile's positions, in a tile with new keys
   __shared__ float mx_l[4][32];   // the first half's row maxima, for the waves of the second
+  extern __shared__ __attribute__((aligned(16))) unsigned char q_l[];
   const RowsLayout r = rows_layout(a);
   const int npair = a.B * a.HK;
   const int id = blockIdx.x, pair = id % npair, grp = (id / npair) % r.ngrp, kt = id / npair / r.ngrp;
@@ -215,7 +231,17 @@ __global__ __launch_bounds__(64 * kSW, 4) void gqa_scores_kernel(GqaArgs a) {
   f4 qwv = {};
   if (tid < kHD / 4) qwv = *(gptr<f4>)(gp<float>(a.qw) + 4 * tid);
   QRow<T> q;
-  q.load(a, b, kh * 4 + hh, q0, half, c32);
+  q.template load<kStaged>(a, b, kh * 4 + hh, q0, half, c32);
+  if constexpr (kStaged) {
+    // 16 of 64 copy instructions a head, two rows each: waves w and w + 4 share head w & 3
+    const char* qg = reinterpret_cast<const char*>(a.in) + ((size_t)b * a.L * a.stride + (size_t)(kh * 4 + hh) * 2 * kHD) * 2;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int ins = 8 * kk + i, rr = 2 * ins + half;
+      dma16(lds_addr(q_l) + hh * 16384 + ins * 1024,
+            (unsigned)min(q0 + rr, a.L - 1) * (unsigned)a.stride * 2u + 16u * (unsigned)(c32 ^ rr), qg);
+    }
+  }
   // cached keys of the tile: 4 of 32 copy instructions a wave, 2 keys each
   if (kt * kBK < a.P) {
     const char* kg = (const char*)(a.K + kvb + (size_t)kt * kBK * kHD);
@@ -263,6 +289,7 @@ __global__ __launch_bounds__(64 * kSW, 4) void gqa_scores_kernel(GqaArgs a) {
     }
   }
   h8 qreg[16];
+  if constexpr (kStaged) q.take(q_l + hh * 16384, half, c32);
   q.load_rope();
   q.prepare(qw_l, half, qreg);
   if (fresh) __syncthreads();  // the new keys are in LDS
@@ -535,9 +562,17 @@ template <typename T>
 hipError_t launch(const GqaArgs& a, hipStream_t s) {
   const RowsLayout r = rows_layout(a);
   const int npair = a.B * a.HK;
-  hipLaunchKernelGGL(gqa_scores_kernel<T>, dim3(npair * r.ngrp * r.nt), dim3(64 * kSW), 0, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  const dim3 grid(npair * r.ngrp * r.nt), block(64 * kSW);
+  hipError_t e;
+  if (sizeof(T) == 2 && a.L > kDirect && grid.x <= 256) {  // (never with f32 rows)
+    if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(gqa_scores_kernel<T, true>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, kQLds)) != hipSuccess)
+      return e;
+    hipLaunchKernelGGL((gqa_scores_kernel<T, true>), grid, block, kQLds, s, a);
+  } else {
+    hipLaunchKernelGGL((gqa_scores_kernel<T, false>), grid, block, 0, s, a);
+  }
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   const int np = a.split > 0 ? (r.nt + a.split - 1) / a.split : 1;
   auto k = a.split > 0 ? gqa_values_kernel<T, true> : gqa_values_kernel<T, false>;
   if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, kVLds)) != hipSuccess)
