@@ -62,13 +62,17 @@ struct ImgOut {
 __device__ __forceinline__ h8 join(const f4& lo, const f4& hi) { return pack_b(lo, hi); }
 
 // ------------------------------------------------------------------------------------------------------------------
-// gdn_prep_kernel: 4 waves. Conv lane pt: rows 8 (pt / 32) .. + 7 of the chunk, channels 4 (pt % 32) .. + 3 of each
+// gdn_prep_kernel. Conv lane pt: rows 4 (pt / 32) .. + 3 of the chunk, channels 4 (pt % 32) .. + 3 of each
 // of q, k and v; q^, k^, k^T and v^T go to LDS. Wave 3 forms the gates, the diagonal blocks of A and their forward
 // substitution; waves 0..2 the six below-diagonal blocks of A and then one block column of T each. The products
 // are then spread over the four waves and written to the image straight from registers.
-constexpr int kPW = 4, kPT = 64 * kPW;
-constexpr int kPRG = 8;  // rows per conv lane
-constexpr int kPG = kPW - 1;
+// 8 waves: wave w + 4 takes half of wave w's tiles where the text below speaks of four waves, and a conv lane 4 rows
+// instead of 8. A workgroup's chain of phases is what bounds the kernel (a few workgroups a CU at most), and the wide ones
+// halve; per element the arithmetic is the same. 4 waves of 8 rows -> this, us a layer: 61 rows after 1531 (B = 1) 25.3 -> 23.5,
+// B = 1, T = 1531 52.0 -> 49.9, T = 4000 104 -> 99; B = 2, T = 2048 97 -> 91.
+constexpr int kHalves = 2, kPT = 256 * kHalves;
+constexpr int kPRG = 8 / kHalves;  // rows per conv lane
+constexpr int kPG = 3;  // the gate wave
 
 // 80,128 bytes, so that two workgroups share a CU (one's row loads overlap the other's arithmetic). The arrays share
 // storage by lifetime: q^ until Att and q~ are written, then A and T (fp32); k^ and the conv taps until A is formed,
@@ -102,7 +106,8 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
   PrepLds& sm = *reinterpret_cast<PrepLds*>(lds_raw);
   const int c = blockIdx.x, bh = blockIdx.y;
   const int b = bh / a.H, h = bh % a.H;
-  const int tid0 = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+  const int tid0 = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+  const int w = wave & 3, hi = wave >> 2;  // hi: which half of wave w's tiles
   const int end = a.P + a.L;
   const int cs = a.s0 + kCH * c;
   const int m = min(kCH, end - cs);
@@ -137,7 +142,7 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
   }
   // the gate wave: a and b of row `lane` of the chunk (rows past the end are masked where the gates are formed)
   float ga = 0.0f, gb = 0.0f;
-  if (w == kPG) {
+  if (wave == kPG) {
     const int lane = tid0 & 63;
     const gptr<T> grow = row_of<T>(a, src, b, min(cs + lane, end - 1));
     ga = (float)grow[aoff];
@@ -189,18 +194,20 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
     }
 #pragma unroll
     for (int cc = 0; cc < 4; cc++) {
-      h8 kt, vt;
+      typedef _Float16 hr __attribute__((ext_vector_type(kPRG)));
+      hr kt, vt;
 #pragma unroll
       for (int r = 0; r < kPRG; r++) {
         kt[r] = (_Float16)(u[r][4 + cc] * rkv[r]);
         vt[r] = (_Float16)u[r][8 + cc];
       }
-      *reinterpret_cast<h8*>(sm.KT + kt16(4 * cl + cc, rg)) = kt;
-      *reinterpret_cast<h8*>(sm.VT + vt16(4 * cl + cc, rg)) = vt;
+      // the lane's part of the 8-row group rg / kHalves
+      *reinterpret_cast<hr*>(sm.KT + kt16(4 * cl + cc, rg / kHalves) + kPRG * (rg % kHalves)) = kt;
+      *reinterpret_cast<hr*>(sm.VT + vt16(4 * cl + cc, rg / kHalves) + kPRG * (rg % kHalves)) = vt;
     }
   }
   // gates: beta, the cumulative log decay (lane = row) and the vectors derived from it
-  if (w == kPG) {
+  if (wave == kPG) {
     const int lane = tid0 & 63;
     float gcr = 0.0f, btr = 0.0f;
     if (lane < m) {
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
   const int lo16 = 16 * lane;
   // Att^T = k^ q^T, decay-masked: tile (a, tb) holds Att[16 tb + c16][16 a + 4 grp + e]; Att block (tb, kb) is the
   // tile pair a = 2 kb, 2 kb + 1 (a tile above the diagonal, a > tb, is zero). The six blocks that are read:
-  // wave 0: (0,0) and (2,1); wave 1: (1,0); wave 2: (2,0); wave 3: (3,0) and (3,1).
+  // waves 0 .. 5: (0,0), (1,0), (2,0), (3,0), (2,1), (3,1).
   {
     auto att_tile = [&](int ta, int tb) {
       const _Float16* ab = sm.Ks + (16 * ta + c16) * kQP + 8 * grp;
@@ -255,24 +262,20 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
       const f4 hi = 2 * kb + 1 <= tb ? att_tile(2 * kb + 1, tb) : z4;
       img.st16(kOffA + (tb * 2 + kb) * kBlk + lo16, join(lo, hi));
     };
-    if (w == 0) {
-      att_block(0, 0);
-      att_block(2, 1);
-    } else if (w == 1) {
-      att_block(1, 0);
-    } else if (w == 2) {
-      att_block(2, 0);
-    } else {
-      att_block(3, 0);
-      att_block(3, 1);
-    }
+    if (wave == 0) att_block(0, 0);
+    if (wave == 1) att_block(1, 0);
+    if (wave == 2) att_block(2, 0);
+    if (wave == 3) att_block(3, 0);
+    if (wave == 4) att_block(2, 1);
+    if (wave == 5) att_block(3, 1);
   }
   // q~ blocks (tb = w, kb 0..3): q^ rows scaled by e^gc, K in the permuted order
   {
     const int t = 16 * w + c16;
     const float eg = sm.eg[t];
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
+    for (int k = 0; k < 4 / kHalves; k++) {
+      const int kb = kHalves * k + hi;
       const h8 q = perm_a(sm.Qs, kQP, t, kb, grp);
       h8 o;
 #pragma unroll
@@ -283,10 +286,10 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
   __syncthreads();  // q^ is dead: A and T reuse its storage
   if (w == kPG) {
     // the four diagonal blocks of A: k^ k^T (A and B operands are the same rows), beta and decay, strictly lower
-    f4 dg[4];
+    f4 dg[4 / kHalves];
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-      const _Float16* kr = sm.Ks + (16 * d + c16) * kQP + 8 * grp;
+    for (int d = 0; d < 4 / kHalves; d++) {
+      const _Float16* kr = sm.Ks + (16 * (kHalves * d + hi) + c16) * kQP + 8 * grp;
       dg[d] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int ks = 0; ks < 4; ks++) {
@@ -295,8 +298,8 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
       }
     }
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-      const int tp = 16 * d + c16, t0 = 16 * d + 4 * grp;
+    for (int d = 0; d < 4 / kHalves; d++) {
+      const int tp = 16 * (kHalves * d + hi) + c16, t0 = 16 * (kHalves * d + hi) + 4 * grp;
       const float gp_ = sm.gc[tp];
       const f4 gt = lds4(&sm.gc[t0]), bv = lds4(&sm.bt[t0]);
 #pragma unroll
@@ -307,9 +310,9 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
       }
     }
   } else {
-    // below-diagonal blocks of A: tiles 1,3,4,6,7,8 of the 10 on or below the diagonal, two per wave
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
+    // below-diagonal blocks of A: tiles 1,3,4,6,7,8 of the 10 on or below the diagonal, one per wave
+    {
+      const int k = hi;
       const int jt = w == 0 ? (k ? 3 : 1) : w == 1 ? (k ? 6 : 4) : (k ? 8 : 7);
       const int ti = jt >= 6 ? 3 : jt >= 3 ? 2 : 1, tj = jt - ti * (ti + 1) / 2;
       const _Float16* ab = sm.Ks + (16 * ti + c16) * kQP + 8 * grp;
@@ -335,7 +338,7 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
     *reinterpret_cast<h8*>(sm.Tb + t * kTP + 8 * g) = h8{};
     *reinterpret_cast<h8*>(sm.Tw + t * kTP + 8 * g) = h8{};
   }
-  if (w == kPG) {
+  if (wave == kPG) {
     // lane (grp, c16): column c16 of diagonal block grp, rows in order (left-looking)
     const int base = 16 * grp;
     float pc[16];
@@ -356,11 +359,11 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
     }
   }
   __syncthreads();
-  if (w == 0)
+  if (wave == 0)
     t_column<0, true>(sm, grp, c16);
-  else if (w == 1)
+  else if (wave == 1)
     t_column<1, true>(sm, grp, c16);
-  else if (w == 2)
+  else if (wave == 2)
     t_column<2, true>(sm, grp, c16);
   __syncthreads();  // T diag(beta), T diag(beta e^gc) complete
 
@@ -368,7 +371,8 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
   // so the tile pair (2w, 2w+1) of one tb is W's A-operand block (tb, kb = w). T is lower triangular: the second
   // K block (chunk rows 32..63) only contributes to tb >= 2.
 #pragma unroll
-  for (int tb = 0; tb < 4; tb++) {
+  for (int tk = 0; tk < 4 / kHalves; tk++) {
+    const int tb = kHalves * tk + hi;
     f4 d[2];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
@@ -387,7 +391,8 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
   }
   // U = T diag(beta) v^: tiles (tb, jt), jt in {2w, 2w+1}, in the D layout
 #pragma unroll
-  for (int tb = 0; tb < 4; tb++) {
+  for (int tk = 0; tk < 4 / kHalves; tk++) {
+    const int tb = kHalves * tk + hi;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const int jt = 2 * w + k;
@@ -404,8 +409,8 @@ __global__ __launch_bounds__(kPT) void gdn_prep_kernel(GdnArgs a) {
     }
   }
   // K~^T blocks (ib in {2w, 2w+1}, kb 0..1): k^ columns with chunk row t scaled by e^(gc_63 - gc_t)
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
+  {
+    const int k = hi;
     const int i = 16 * (2 * w + k) + c16;
 #pragma unroll
     for (int kb = 0; kb < 2; kb++) {
