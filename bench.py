@@ -302,12 +302,12 @@ def mnb_measure(torch, ha, stream, steps=20, Ms=MNB_MS):
         d = {"ms_per_forward": round(p["ms"], 4), "us_per_call": p["shapes"]}
         if M == 1:
             gbs = p["bytes"] / (p["ms"] * 1e-3) / 1e9
-            d["roofline"] = {"bound": "hbm", "kernel": "mnb_gemv_lanes_kernel", "achieved": round(gbs, 1),
+            d["roofline"] = {"bound": "hbm", "kernel": "mnb_strip_kernel, mnb_gemv_lanes_kernel", "achieved": round(gbs, 1),
                              "peak": 8000.0, "unit": "GB/s", "frac": round(gbs / 8000.0, 4),
                              "bytes_per_forward": p["bytes"], "traffic": None}
         else:
             tf = p["flops"] / (p["ms"] * 1e-3) / 1e12
-            d["roofline"] = {"bound": "mfma", "kernel": "mnb_gemm_kernel",
+            d["roofline"] = {"bound": "mfma", "kernel": "mnb_tiles_kernel, mnb_strip_kernel",
                              "achieved": round(tf, 1), "peak": 2500.0, "unit": "TFLOP/s",
                              "frac": round(tf / 2500.0, 4), "flops_per_forward": p["flops"], "traffic": None}
         out["M%d" % M] = d
