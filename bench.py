@@ -191,7 +191,7 @@ def decode_measure(torch, ha, stream, steps=50, P=1536):
     then calls of L new rows resumed from it, each timed alone (HIP events on the engine's stream around one call,
     median over `steps`).
       gdn_seq   one gated-delta layer, L = 1 and 8 rows, HA_SEQUENTIAL, B = 1 and 8: GB/s against the algorithmic
-                bytes (fp32 state in and out, 64 KiB each per head, plus the rows read and written)
+                bytes (the fp32 state in, 64 KiB per head, plus the rows read and written; no snapshot is kept, so no state out)
       stack     the 24-layer stack at B = 1 and 8, L = 1 (sequential recurrence for the gated-delta layers)
       resume    the prefix-cache case: 3 gated-delta + 1 GQA layers, one 64-row suffix at P = 1536 (B = 1, default
                 recurrence), with and without keeping a snapshot of the result"""
@@ -217,7 +217,7 @@ def decode_measure(torch, ha, stream, steps=50, P=1536):
         for L in (1, 8):
             si, so = make_buffers(torch, ["linear_attention"], B, L, seed=8)
             ms = timed(lambda: eng.forward(L, si, so, cache=snap, recurrence=ha.SEQUENTIAL))
-            byt = B * (2 * H * DK * DV * 4 + L * gdn_bytes_per_token())
+            byt = B * (H * DK * DV * 4 + L * gdn_bytes_per_token())
             res["gdn_seq_B%d_L%d" % (B, L)] = {"us": round(ms * 1e3, 2), "GB_per_s": round(byt / (ms * 1e-3) / 1e9, 1),
                                                "bytes": byt, "frac": round(byt / (ms * 1e-3) / 8e12, 4)}
             del si, so
