@@ -106,13 +106,18 @@ __global__ __launch_bounds__(64 * WM * WN, kMinWaves) void mnb_tiles_kernel(MnbA
 #pragma unroll
     for (int c = 0; c < CT; c++) acc[i][c] = f16v{};
   const unsigned arow = (unsigned)(32 * RT * wm + fr) * 128u;
-  // Tile kt, in stage kt % 3, its weights in registers kt % 2. Loads complete in order: taking the weights of tile kt into
-  // use (issued after the copy of a tile kt + 1) also waits for this wave's part of that copy, a whole tile's time after it
-  // was issued; the barrier at the end then makes tile kt + 1 everybody's. The copy of tile kt + 2 goes into the stage that
-  // tile kt - 1 left before the last barrier.
+  // Tile kt, in stage kt % 3, its weights in registers kt % 2. Loads complete in order: in flight at the top are the weights of
+  // tile kt, this wave's part of the copy of tile kt + 1 (a whole tile's time old) and the weights of tile kt + 1, so waiting
+  // for all but the last kWLoads lands the first two; the barrier at the end then makes tile kt + 1 everybody's. The wait is
+  // written out: the compiler's own, for the weights, is none in a wave that uses no weights. The copy of tile kt + 2 goes
+  // into the stage that tile kt - 1 left before the last barrier.
   auto step = [&](int kt, int stage, int q) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWLoads) : "memory");
 #pragma unroll
-    for (int c = 0; c < CT; c++) asm volatile("" : "+v"(wr[q][c]), "+v"(sr[q][c])::"memory");
+    for (int c = 0; c < CT; c++) {
+      asm volatile("" : "+v"(wr[q][c]), "+v"(sr[q][c])::"memory");
+      if constexpr (ASYM) asm volatile("" : "+v"(br[q][c])::"memory");
+    }
     copy_a(kt + 2, (stage + 2) % kStages);
     if (active) {
       const unsigned char* as = sm + stage * kStage + arow;

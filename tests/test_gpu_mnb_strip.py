@@ -59,11 +59,13 @@ def test_tile_edges(N, K, bits, group, asym):
 
 
 @pytest.mark.parametrize("N,K,group,asym", [
-    (4160, 192, 32, False), (4112, 448, 32, True), (3008, 1024, 64, False), (8256, 128, 64, True), (5120, 64, 32, False)])
+    (4160, 192, 32, False), (4112, 448, 32, True), (3008, 1024, 64, False), (8256, 128, 64, True), (5120, 64, 32, False),
+    (3008, 384, 64, True), (2208, 384, 32, True), (4256, 384, 64, False), (4256, 2048, 32, True), (2208, 2048, 64, True)])
 def test_many_rows(N, K, group, asym):
-    # more rows than the strip kernel is the faster for: the tile kernel, at edges of its tiles in both directions (a last
-    # column tile of 16, 64, 192 and 256; rows just over and under a multiple of 128 and 256) and of its six-tile K loop;
-    # rows keep their bits whatever M is
+    # more rows than the strip kernel is the faster for: the tile kernel, at edges of its tiles in both directions (rows just
+    # over and under a multiple of 128 and 256; last column tiles of 32, 64, 160, 192 and 256 columns, so that some waves have
+    # none, while the up to 64 columns past a multiple of 256 of 4112, 4160 and 8256 go to the strip kernel) and of its
+    # six-tile K loop; rows keep their bits whatever M is
     import torch
     words, sc, bi = _weights(N, K, 4, group, asym, N + K)
     W = mo.dequant(words, sc, N, K, 4, group, asym, bi)
