@@ -85,7 +85,7 @@ struct Scratch {
   int device = 0;
   Buf img, seq_raw, seq_cnt, gqa_part, gqa_rows, gqa_marks, zeros, duo_ring, sync_flags;
   unsigned sync_epoch = 0;  // the progress counters' epoch of the last launch that used them (they start at zero)
-  unsigned gqa_epoch = 0;   // the GQA marks' epoch of the last launch (the marks start at zero)
+  unsigned gqa_epoch = 0;   // the split-GQA slot marks' epoch of the last launch (the marks start at zero)
   // the engines holding this set (guarded by g_live_mu); all of them run on one stream, so their calls never overlap
   std::vector<const ha_engine*> holders;
   ~Scratch() {
@@ -782,20 +782,23 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       a.split = e->gqa_split; a.part_slots = e->gqa_part_slots; a.part = static_cast<float*>(sc.gqa_part.p);
       a.rows = sc.gqa_rows.p; a.row_marks = static_cast<unsigned*>(sc.gqa_marks.p);
       const bool rows = ha::gqa_rows_takes(a);
-      if (a.split > 0 || rows) {
+      if (a.split > 0 && !rows) {
         // a fresh mark per launch; if the counter wraps, the marks (and partials) are cleared first
         if (++sc.gqa_epoch == 0) {
           HA_HIP(hipStreamSynchronize(st));
-          if (sc.gqa_part.p) HA_HIP(hipMemset(sc.gqa_part.p, 0, sc.gqa_part.bytes));
-          HA_HIP(hipMemset(sc.gqa_marks.p, 0, sc.gqa_marks.bytes));
+          HA_HIP(hipMemset(sc.gqa_part.p, 0, sc.gqa_part.bytes));
           sc.gqa_epoch = 1;
         }
         a.epoch = sc.gqa_epoch;
       }
-      // the merge waits for marks equal to this launch's epoch: epoch + 1 is never written by it
+      // the waits are for marks equal to this launch's epoch, or to one in a short call: the next value is never written
       a.wait = wait;
       if (unpublished) a.wait.skew = 1u;
       hipError_t he = rows ? ha::launch_gqa_rows(a, st) : ha::launch_gqa(a, st);
+      if (he != hipSuccess && rows) {  // the second launch, which clears the marks, may be the one that failed
+        (void)hipStreamSynchronize(st);
+        (void)hipMemset(sc.gqa_marks.p, 0, sc.gqa_marks.bytes);
+      }
       if (he != hipSuccess) return fail(HA_ERR_DEVICE, "layer " + std::to_string(i) + " attention launch: " + hipGetErrorString(he));
       if (per_layer) HA_HIP(hipEventRecord(e->mev[i], st));
     } else if (per_layer) {  // HA_ADAPTER: no token mixer, nothing to run

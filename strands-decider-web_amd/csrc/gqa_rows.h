@@ -40,7 +40,9 @@ constexpr int kMUnit = 32 * 4;   // bytes of a half's row maxima, and of its ref
 
 // Scratch of a call: per chain unit u = ((pair * ngrp + group) * 4 + head) * nh + half all P, then all statistics, all
 // maxima, all reference maxima. The marks [pair][group][tile] are a buffer of their own, so that no other data ever lies where a mark is
-// looked for.
+// looked for. They are zero between calls: a scores workgroup sets its own, the values kernel clears them again, so a
+// launch that a graph replays waits for its own marks and not for those of the replay before.
+constexpr unsigned kMark = 1;
 struct RowsLayout {
   int ngrp, nt, nh;  // query groups, tiles of the longest group, halves
   unsigned units;    // chain units in all
@@ -329,14 +331,14 @@ __global__ __launch_bounds__(64 * kSW, 4) void gqa_scores_kernel(GqaArgs a) {
   if (kk == 0 && half == 0) mx_l[hh][c32] = mx;
   __builtin_amdgcn_s_waitcnt(0);  // this wave's maxima have reached the device-coherent level
   __syncthreads();                // ... and every wave's
-  if (tid == 0) __hip_atomic_store(marks + kt, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) __hip_atomic_store(marks + kt, kMark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   float mref = -INFINITY;
   auto raise = [&](float m) { mref = m > mref + kRescale ? m : mref; };
   if (first < kt) {
     if (w == 0) {
       // bounded; a wait that runs out is reported through the engine's error word (a test's skew makes every mark this
       // wait looks for one that no workgroup writes)
-      const unsigned want = a.epoch + a.wait.skew;
+      const unsigned want = kMark + a.wait.skew;
       for (int j0 = first; j0 < kt; j0 += 64) {
         const int j = min(j0 + lane, kt - 1);
         int i = 0;
@@ -556,6 +558,10 @@ __global__ __launch_bounds__(kSplit ? 64 * kMaxPieces : 256) void gqa_values_ker
     asm volatile("" : "+v"(y));  // rounded to f32 before f16, as gqa_attn_kernel rounds it, not by one mixed-precision fma
     if (t < a.L) gpw<T>(a.out)[((size_t)b * a.L + t) * (size_t)(a.HQ * kHD) + d] = (T)y;
   }
+  // every scores workgroup has ended: its pair's and group's marks are cleared for the next call
+  if (sl == 0 && w == 0 && (!kSplit || hh == 0))
+    for (int j = lane; j < r.nt; j += 64)
+      __hip_atomic_store(a.row_marks + ((size_t)pair * r.ngrp + grp) * r.nt + j, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <typename T>
@@ -608,7 +614,7 @@ bool gqa_rows_takes(const GqaArgs& a) {
 }
 
 hipError_t launch_gqa_rows(const GqaArgs& a, hipStream_t s) {
-  if (!gqa_rows_takes(a) || a.epoch == 0 || a.P + a.L > a.LT) return hipErrorInvalidValue;
+  if (!gqa_rows_takes(a) || a.P + a.L > a.LT) return hipErrorInvalidValue;
   if (a.split > 0 && (a.LT / kBK + a.split - 1) / a.split > gqa_rows::kMaxPieces) return hipErrorInvalidValue;
   // maxima are addressed by 32-bit byte offsets
   if ((size_t)gqa_rows::rows_layout(a).units * gqa_rows::kMUnit > 0x7fffffff) return hipErrorInvalidValue;

@@ -79,9 +79,9 @@ struct GqaArgs {
   int part_slots;
   float* part;               // [slots][4][64][HD] unnormalised O, then [slots][4][64][2] (reference max, sum), then
                              // [slots] u32 epoch marks
-  unsigned epoch;            // this launch's mark, >= 1 and different from every earlier launch's on `part` or `row_marks`
+  unsigned epoch;            // split key ranges: this launch's mark, >= 1 and different from every earlier launch's on `part`
   void* rows;                // short calls: scratch of gqa_rows_bytes(), or nullptr
-  unsigned* row_marks;       // short calls: gqa_rows_marks() marks
+  unsigned* row_marks;       // short calls: gqa_rows_marks() marks, zero between calls
   WaitCheck wait;            // the merge workgroups' bounded wait for their pieces
 };
 
