@@ -570,7 +570,9 @@ hipError_t launch(const GqaArgs& a, hipStream_t s) {
   const int npair = a.B * a.HK;
   const dim3 grid(npair * r.ngrp * r.nt), block(64 * kSW);
   hipError_t e;
-  if (sizeof(T) == 2 && a.L > kDirect && grid.x <= 256) {  // (never with f32 rows)
+  // the staging copies move 16 bytes at a time: rows that are not 16-byte aligned are read directly
+  const bool aligned = a.stride % 8 == 0 && (uintptr_t)a.in % 16 == 0;
+  if (sizeof(T) == 2 && a.L > kDirect && grid.x <= 256 && aligned) {  // (never with f32 rows)
     if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(gqa_scores_kernel<T, true>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, kQLds)) != hipSuccess)
       return e;

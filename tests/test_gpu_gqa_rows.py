@@ -37,6 +37,32 @@ def test_rows_equal_a_long_forward(B, P, steps, f32):
         np.testing.assert_array_equal(got, want[:, :, :a], err_msg=part)
 
 
+@pytest.mark.parametrize("stride,off", [(5124, 0), (5120, 4), (5132, 4)])
+def test_rows_that_are_not_16_byte_aligned(stride, off):
+    # a row stride or a first row at a multiple of 8 bytes only: the same bits as 16-byte aligned rows
+    import torch
+    x = torch.from_numpy(synth.gqa_rows(300, 1, seed=33)).to("cuda:0")
+    outs = []
+    for st, of in ((5120, 0), (stride, off)):
+        e = ha.Engine(ha.model_config(["full_attention"], batch=1, max_ctx=512, full_stride=st))
+        for n, v in synth.gqa_params(seed=33, noise=0.1).items():
+            e.set_param(0, n, v)
+        buf = torch.zeros(300 * st + of + 8, dtype=torch.float16, device="cuda:0")
+        rows = buf[of:of + 300 * st].view(300, st)
+        rows[:, :5120] = x[0]
+        o = torch.empty(1, 300, 2048, dtype=torch.float16, device="cuda:0")
+        torch.cuda.synchronize()
+        snap = e.forward(200, [rows], [o], keep_cache=True, sync=True)["cache"]
+        for a, b in ((200, 261), (200, 209)):
+            o2 = torch.empty(1, b - a, 2048, dtype=torch.float16, device="cuda:0")
+            torch.cuda.synchronize()
+            e.forward(b - a, [rows[a:]], [o2], cache=snap, sync=True)
+            outs.append((st, of, o2))
+        outs.append((st, of, o[:, :200].clone()))
+    for (_, _, w), (_, _, g) in zip(outs[:3], outs[3:]):
+        assert torch.equal(w, g)
+
+
 def test_wait_that_runs_out_is_reported():
     import torch
     x = torch.from_numpy(synth.gqa_rows(200, 1, seed=32)).to("cuda:0")
