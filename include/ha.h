@@ -175,7 +175,8 @@ int ha_snapshot_layout(const ha_snapshot* s, int* state_pos, int* tail_rows);
                     (a resume replays those rows in the chunked form instead, so that prefix + suffix stays
                     bit-identical to one forward; the two agree within the recurrence tolerance)
      "state_stored" f32 [batch][H][DK][DV]: the stored state at state_pos (what a resume starts from)
-     "tail"         [batch][tail_rows][lin_stride] in lin_dtype: the raw rows [state_pos - (conv_k-1), P)
+     "tail"         [batch][tail_rows][lin_stride] in lin_dtype: the raw rows [state_pos - (conv_k-1), P), of which the
+                    conv channels (q | k | v) and the a and b columns are kept; z and the padding read as zero
      "K" / "V"      f16 [batch][HK][P][HD]. */
 int ha_snapshot_read(const ha_snapshot* s, int layer, const char* what, void* host, size_t bytes);
 /* Free the snapshot's device memory (snapshot.release(), engine.js:361). Idempotent. */

@@ -1,8 +1,10 @@
 // Raw-row tail of a gated-delta layer, gfx950: the generalisation of the reference's conv history roll
 // (HIST_UPDATE, web/public/engine/wgsl.js:420-434). After a call, the rows [state_pos - 3, P + L) are kept so that
 // the next call can rebuild the conv history and replay the rows after the stored state position. Only the conv
-// channels and the a/b gate columns are copied (z is not needed for replay). The copy reads only the call's input
-// rows and the tail it resumed from, never a mixer's output, so one launch serves every gated-delta layer of a call.
+// channels and the a/b gate columns are copied (z is not needed for replay); the others are cleared, since the rows go
+// straight into a snapshot's block, which may hold an earlier snapshot's data, and a host can read them. The copy reads
+// only the call's input rows and the tail it resumed from, never a mixer's output, so one launch serves every
+// gated-delta layer of a call.
 #include "ha_kernels.h"
 
 namespace ha {
@@ -24,6 +26,8 @@ __global__ __launch_bounds__(256) void tail_update_kernel(TailArgs a) {
   const U* s2 = reinterpret_cast<const U*>(src + a.ab_off);
   U* d2 = reinterpret_cast<U*>(dst + a.ab_off);
   for (int c = threadIdx.x; c < a.ab_n / kPer; c += blockDim.x) d2[c] = s2[c];
+  for (int c = a.C / kPer + threadIdx.x; c < a.ab_off / kPer; c += blockDim.x) d1[c] = U{};
+  for (int c = (a.ab_off + a.ab_n) / kPer + threadIdx.x; c < a.stride / kPer; c += blockDim.x) d1[c] = U{};
 }
 
 struct alignas(16) U16 {

@@ -7,6 +7,7 @@ conv history."""
 import numpy as np
 import pytest
 
+import hybrid_attention as ha
 import synth
 from harness import Runner
 
@@ -33,3 +34,24 @@ def test_many_layer_tails_resume_bit_exact(batch, layer_ms):
         assert np.isfinite(outs[i]).all(), i
         np.testing.assert_array_equal(outs[i], full[i][:, 100:], err_msg="layer %d" % i)
     snap.release()
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_tail_reads_the_rows_and_zeros(f16):
+    # the raw rows of a snapshot as a host reads them: conv channels, a and b as they came in, the other columns zero, and the
+    # same bytes in a block whose place of the rows held an earlier snapshot's K and V (three raw rows, then 1920 positions)
+    B, C, AB = 2, 6144, 8192
+    dt = np.float16 if f16 else np.float32
+    r = Runner(["linear_attention", "full_attention"], batch=B, lin_dtype=ha.F16 if f16 else ha.F32)
+    r.set_params(0, synth.gdn_params(seed=6))
+    x = [synth.gdn_rows(180, B, seed=6).astype(dt), synth.gqa_rows(180, B, seed=6)]
+    for n in range(2):
+        _, snap = r.forward(x, keep=True)
+        assert (snap.state_pos, snap.tail_rows) == (128, 55)
+        g = snap.read(0, "tail", np.full((B, 55, 8256), 3, dt))
+        np.testing.assert_array_equal(g[..., :C], x[0][:, 125:, :C])
+        np.testing.assert_array_equal(g[..., AB:AB + 32], x[0][:, 125:, AB:AB + 32])
+        assert not g[..., C:AB].any() and not g[..., AB + 32:].any(), n
+        if n == 0:  # a larger block, which the next snapshot takes (the engine keeps one released block)
+            _, large = r.forward([synth.gdn_rows(1920, B, seed=7).astype(dt), synth.gqa_rows(1920, B, seed=7)], keep=True)
+            large.release()
