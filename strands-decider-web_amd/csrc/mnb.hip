@@ -163,14 +163,21 @@ __global__ __launch_bounds__(64 * kGW) void mnb_gemv_kernel(MnbArgs a) {
   }
 }
 
-// y for M = MR <= 2 rows: a wave owns LW consecutive output columns and its lanes run along K. Lane l takes blocks l,
+// y for M = MR <= 2 rows: a wave owns a few consecutive output columns and its lanes run along K. Lane l takes blocks l,
 // l + 64, ... of each of its columns (one whole-block load per column, so a wave instruction reads a contiguous 1 KiB of
 // one column's packed row), dequantises them and multiplies them into the rows of a with v_dot2_f32_f16 (fp32
-// accumulation); the next blocks are loaded before the current ones are used. The lanes' partial sums are added by DPP and
-// permlane. Bound: round trips, in a kernel of a few us. With two columns a wave the rows of a come through LDS, copied once
-// per workgroup in whole lines while the first blocks are on their way: read directly, a lane's 64 bytes are a cache line
-// of their own, twice the address cycles of two columns' weights. With four the copy and its barrier cost more than it
-// saves. Grid: N / (4 LW) workgroups of 4 waves. 2048 x 6144: 6.1 -> 5.1 us with one row, 7.4 -> 5.6 with two (LW = 4 -> 2).
+// accumulation). The lanes' partial sums are added by DPP and permlane. Bound: round trips, in a kernel of a few us. Two
+// forms:
+//   two columns a wave (launch_lanes: below kLaneWide columns): the next blocks are loaded before the current ones are
+//     used, and the rows of a come through LDS, copied once per workgroup in whole lines while the first blocks are on
+//     their way: read directly, a lane's 64 bytes are a cache line of their own, twice the address cycles of two columns'
+//     weights. 2048 x 6144, weights rotating through eight matrices: 6.1 us with four columns a wave, 4.9 with two; two
+//     rows 7.3 and 5.0.
+//   four columns a wave (mnb_gemv_wide_kernel): twice the arithmetic for each load of a, which is read directly; staged,
+//     the copy and its barrier cost more than they save.
+// Scales are held in whole registers: as an array of 16-bit values the compiler kept them in memory (scratch, or LDS read
+// at odd addresses, which took 17 us at 4096 x 2048 against 4.3).
+// Grid: a workgroup for 4 waves' columns.
 constexpr int kLaneChunk = 8192;  // k of a in LDS at a time
 __device__ __forceinline__ float lanes_sum(float v) {
   auto ror = [](float x, auto ctrl) {
@@ -187,21 +194,20 @@ __device__ __forceinline__ float lanes_sum(float v) {
   const auto q = __builtin_amdgcn_permlane32_swap(t, t, false, false);
   return __builtin_bit_cast(float, (unsigned)q[0]) + __builtin_bit_cast(float, (unsigned)q[1]);
 }
-template <int BITS, int GROUP, bool ASYM, int MR, int LW>
+template <int BITS, int GROUP, bool ASYM, int MR>
 __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char al[];  // [row][16-byte chunks], chunk q at q ^ (q / 16 % 4)
-  const int tid = threadIdx.x, lane = tid & 63, n0 = LW * (4 * blockIdx.x + (tid >> 6));
+  constexpr int kLW = 2;
+  const int tid = threadIdx.x, lane = tid & 63, n0 = kLW * (4 * blockIdx.x + (tid >> 6));
   const int nblk = a.K / kBlk, ng = a.K / GROUP;
-  constexpr bool kStaged = LW == 2;
-  const int chunk = kStaged ? kLaneChunk : a.K;
   struct Blk {
-    unsigned wd[LW][BITS];
-    unsigned short sc[LW], bi[LW];
+    unsigned wd[kLW][BITS];
+    unsigned sc[kLW], bi[kLW];  // f16 bits
   };
   auto load = [&](int b, Blk& x) {
     b = min(b, nblk - 1);
 #pragma unroll
-    for (int c = 0; c < LW; c++) {
+    for (int c = 0; c < kLW; c++) {
       gptr<unsigned> wp = gp<unsigned>(a.q) + ((size_t)(n0 + c) * nblk + b) * BITS;
 #pragma unroll
       for (int j = 0; j < BITS; j++) x.wd[c][j] = wp[j];
@@ -210,9 +216,9 @@ __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
       x.bi[c] = ASYM ? gp<unsigned short>(a.b)[gi] : 0;
     }
   };
-  float acc[LW][MR];
+  float acc[kLW][MR];
 #pragma unroll
-  for (int c = 0; c < LW; c++)
+  for (int c = 0; c < kLW; c++)
 #pragma unroll
     for (int m = 0; m < MR; m++) acc[c][m] = 0.0f;
   auto use = [&](int b, int k0, const Blk& x) {
@@ -222,11 +228,10 @@ __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const int q = 4 * (b - k0 / kBlk) + j;
-        if constexpr (!kStaged) av[m][j] = *(gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + (size_t)b * kBlk + 8 * j);
-        else av[m][j] = *reinterpret_cast<const h8*>(al + (size_t)m * 2 * min(a.K, kLaneChunk) + 16 * (q ^ ((q >> 4) & 3)));
+        av[m][j] = *reinterpret_cast<const h8*>(al + (size_t)m * 2 * min(a.K, kLaneChunk) + 16 * (q ^ ((q >> 4) & 3)));
       }
 #pragma unroll
-    for (int c = 0; c < LW; c++) {
+    for (int c = 0; c < kLW; c++) {
       const h2 sc = splat2u(x.sc[c]), bi = splat2u(x.bi[c]);
 #pragma unroll
       for (int j = 0; j < 4; j++) {
@@ -244,17 +249,15 @@ __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
   };
   Blk cur;
   load(lane, cur);
-  for (int k0 = 0; k0 < a.K; k0 += chunk) {
-    const int n = min(a.K - k0, chunk);
-    if constexpr (kStaged) {
-      if (k0) __syncthreads();  // the chunk before has been read
+  for (int k0 = 0; k0 < a.K; k0 += kLaneChunk) {
+    const int n = min(a.K - k0, kLaneChunk);
+    if (k0) __syncthreads();  // the chunk before has been read
 #pragma unroll
-      for (int m = 0; m < MR; m++)
-        for (int q = tid; q < n / 8; q += 256)
-          *reinterpret_cast<h8*>(al + (size_t)m * 2 * min(a.K, kLaneChunk) + 16 * (q ^ ((q >> 4) & 3))) =
-              *(gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + k0 + 8 * q);
-      __syncthreads();
-    }
+    for (int m = 0; m < MR; m++)
+      for (int q = tid; q < n / 8; q += 256)
+        *reinterpret_cast<h8*>(al + (size_t)m * 2 * min(a.K, kLaneChunk) + 16 * (q ^ ((q >> 4) & 3))) =
+            *(gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + k0 + 8 * q);
+    __syncthreads();
     for (int b = k0 / kBlk + lane; b < (k0 + n) / kBlk; b += 64) {
       Blk next;
       load(b + 64, next);
@@ -263,7 +266,59 @@ __global__ __launch_bounds__(256) void mnb_gemv_lanes_kernel(MnbArgs a) {
     }
   }
 #pragma unroll
-  for (int c = 0; c < LW; c++)
+  for (int c = 0; c < kLW; c++)
+#pragma unroll
+    for (int m = 0; m < MR; m++) {
+      const float v = lanes_sum(acc[c][m]);
+      if (lane == 0 && m < a.M) ((_Float16*)a.y)[(size_t)m * a.N + n0 + c] = (_Float16)v;
+    }
+}
+
+template <int BITS, int GROUP, bool ASYM, int MR>
+__global__ __launch_bounds__(256) void mnb_gemv_wide_kernel(MnbArgs a) {
+  constexpr int kLW = 4;
+  const int lane = threadIdx.x & 63, n0 = kLW * (4 * blockIdx.x + (threadIdx.x >> 6));
+  const int nblk = a.K / kBlk, ng = a.K / GROUP;
+  float acc[kLW][MR];
+#pragma unroll
+  for (int c = 0; c < kLW; c++)
+#pragma unroll
+    for (int m = 0; m < MR; m++) acc[c][m] = 0.0f;
+  for (int b = lane; b < nblk; b += 64) {
+    unsigned wd[kLW][BITS];
+    h2 sc[kLW], bi[kLW];
+#pragma unroll
+    for (int c = 0; c < kLW; c++) {
+      gptr<unsigned> wp = gp<unsigned>(a.q) + ((size_t)(n0 + c) * nblk + b) * BITS;
+#pragma unroll
+      for (int j = 0; j < BITS; j++) wd[c][j] = wp[j];
+      const size_t gi = (size_t)(n0 + c) * ng + b * kBlk / GROUP;
+      sc[c] = splat2(gp<_Float16>(a.s)[gi]);
+      bi[c] = splat2(ASYM ? gp<_Float16>(a.b)[gi] : (_Float16)0.0f);
+    }
+    h8 av[MR][4];
+#pragma unroll
+    for (int m = 0; m < MR; m++) {
+      gptr<h8> ap = (gptr<h8>)(gp<_Float16>(a.a) + (size_t)min(m, a.M - 1) * a.K + (size_t)b * kBlk);
+#pragma unroll
+      for (int j = 0; j < 4; j++) av[m][j] = perm8(ap[j]);
+    }
+#pragma unroll
+    for (int c = 0; c < kLW; c++) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const h8 wv = dequant8_pk<BITS, ASYM>(wd[c], j, sc[c], bi[c]);
+#pragma unroll
+        for (int m = 0; m < MR; m++)
+#pragma unroll
+          for (int p = 0; p < 4; p++)
+            acc[c][m] = __builtin_amdgcn_fdot2(h2{av[m][j][2 * p], av[m][j][2 * p + 1]}, h2{wv[2 * p], wv[2 * p + 1]},
+                                               acc[c][m], false);
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < kLW; c++)
 #pragma unroll
     for (int m = 0; m < MR; m++) {
       const float v = lanes_sum(acc[c][m]);
@@ -546,13 +601,14 @@ void launch_fwht_log(_Float16* x, long blocks, float scale, hipStream_t s) {
   hipLaunchKernelGGL(fwht_kernel<LOG>, dim3((unsigned)((blocks + kPer - 1) / kPer)), dim3(kWG), 0, s, x, blocks, scale);
 }
 
+constexpr int kLaneWide = 4096;  // columns
 template <int BITS, int GROUP, bool ASYM, int MR>
 void launch_lanes(const MnbArgs& a, hipStream_t s) {
-  if (a.N < 4096)
-    hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, MR, 2>), dim3(a.N / 8), dim3(256),
+  if (a.N < kLaneWide)
+    hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, MR>), dim3(a.N / 8), dim3(256),
                        (size_t)MR * 2 * std::min(a.K, kLaneChunk), s, a);
   else
-    hipLaunchKernelGGL((mnb_gemv_lanes_kernel<BITS, GROUP, ASYM, MR, 4>), dim3(a.N / 16), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((mnb_gemv_wide_kernel<BITS, GROUP, ASYM, MR>), dim3(a.N / 16), dim3(256), 0, s, a);
 }
 template <int BITS, int GROUP, bool ASYM>
 hipError_t launch_gemv_lanes(const MnbArgs& a, hipStream_t s) {
