@@ -215,7 +215,7 @@ int ha_mnb_create(int N, int K, const ha_mnb_format* fmt, const void* q, const v
 /* y[M][N] = a[M][K] x W^T (f16 in and out, fp32 accumulation) on `stream` (hipStream_t as void*, NULL: the null
    stream): the matmul dispatch of engine.js:236-246, kernel chosen by M as engine.js:17-33 does. a and y are device
    pointers (16-byte aligned). Operands whose K is a multiple of 64 (128 with groups of 64), with q 16-byte (2 and 3
-   bits: 4-byte) and s, b 4-byte aligned, need no workspace with 4 bits, nor up to 384 rows with 2 and 3. Other products
+   bits: 4-byte) and s, b 4-byte aligned, need no workspace with 4 bits, nor up to 64 rows with 2 and 3. Other products
    with few output tiles split K over workgroups, using a workspace the handle owns (grown on demand, at most 64 MiB), so
    calls on one handle must be ordered. */
 int ha_mnb_forward(ha_mnb* w, int M, const void* a, void* y, void* stream);

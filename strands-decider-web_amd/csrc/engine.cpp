@@ -1049,13 +1049,13 @@ int mnb_forward(ha_mnb* w, int M, const void* a, void* y, void* stream, bool noa
   ha::MnbArgs g = w->args;
   g.M = M; g.a = a; g.y = y;
   g.ldy = g.N;
-  switch (ha::mnb_path(g)) {
+  switch (ha::mnb_path(ha::mnb_shape(g))) {
     case ha::kMnbGemv: HA_HIP(ha::launch_mnb_gemv(g, st)); return HA_OK;
     case ha::kMnbStrip: HA_HIP(ha::launch_mnb_strip(g, st)); return HA_OK;
     case ha::kMnbTiles: HA_HIP(ha::launch_mnb_tiles(g, st)); return HA_OK;
     case ha::kMnbGemm: break;
   }
-  g.split = ha::mnb_gemm_split(M, g.N, g.K);
+  g.split = ha::gemm::split(M, g.N, g.K);
   if (g.split > 1 && noalloc) {
     const size_t need = sizeof(float) * (size_t)g.split * M * g.N;
     if (need > ha::kMnbScratchBytes)

@@ -4,6 +4,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "mnb_plan.h"
+
 namespace ha {
 
 // Cross-workgroup waits of one launch (the paired form's tile-set wait, the split form's packed-state wait, the split
@@ -132,15 +134,11 @@ struct MnbArgs {
 };
 hipError_t mnb_check(const MnbArgs& a);
 bool mnb_strip_takes(const MnbArgs& a);     // whether launch_mnb_strip can run these operands (K, alignment)
-float mnb_strip_us(const MnbArgs& a);       // the time it is expected to take
 hipError_t launch_mnb_strip(const MnbArgs& a, hipStream_t s);
 bool mnb_tiles_takes(const MnbArgs& a);     // likewise launch_mnb_tiles (4-bit weights)
-float mnb_tiles_us(const MnbArgs& a);
 hipError_t launch_mnb_tiles(const MnbArgs& a, hipStream_t s);
-enum MnbPath { kMnbGemv, kMnbStrip, kMnbTiles, kMnbGemm };
-MnbPath mnb_path(const MnbArgs& a);         // the kernel that serves a call
+MnbShape mnb_shape(const MnbArgs& a);        // what mnb_path chooses the kernel by
 hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s);  // M <= 64
-int mnb_gemm_split(int M, int N, int K);  // K ranges the GEMM uses for this shape (1: none, no workspace)
 hipError_t launch_mnb_gemm(const MnbArgs& a, hipStream_t s);  // any M: tiled GEMM, weights dequantised into LDS
 // Scratch of the allocation-free GEMM entry point (mnb.hip): a file-scope device array of kMnbScratchBytes per GPU.
 // mnb_scratch_setup looks its address up on `device`, which must be current, once per device; mnb_scratch returns

@@ -10,12 +10,12 @@
 //   hold the low two bits as in the 2-bit layout and bit e of word 2 is element e's high bit. One f16 scale per
 //   `group` (32 or 64) values of a row; symmetric w = (q - 2^(bits-1)) * scale, asymmetric w = q * scale + bias.
 //
-// Implementations, chosen by M as the reference chooses its kernels by M (mnb_path):
-//   M <= 2    mnb_gemv_lanes_kernel (below 4096 columns): a wave owns 2 output columns, its lanes run along K over
-//             whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
+// Implementations, chosen by M as the reference chooses its kernels by M (mnb_path, mnb_plan.h):
+//   M <= 2    mnb_gemv_lanes_kernel, mnb_gemv_wide_kernel (narrow matrices, and very large ones): a wave owns 2 or 4 output
+//             columns, its lanes run along K over whole packed blocks, v_dot2_f32_f16 products, a cross-lane reduction.
 //   few rows  mnb_strip_kernel (mnb_strip.h): each wave of a workgroup takes a part of K through LDS of its own.
 //   many rows mnb_tiles_kernel (mnb_tiles.h, 4 bits): MFMA tiles, weights dequantised in registers.
-// and for operands that do not suit the DMAs of those two (K % 64, alignment), or 2 and 3 bits above 384 rows:
+// and for operands that do not suit the DMAs of those two (K % 64, alignment), or 2 and 3 bits with many rows or columns:
 //   M <= 64   mnb_gemv_kernel: a workgroup owns 16 output columns and its 8 waves split the K blocks; each lane
 //             dequantises a whole packed block into the f16 B operands of v_mfma_f32_16x16x32_f16 (no LDS), the a rows
 //             are the A operand (16 rows per tile, up to 4 tiles share each dequantised operand), and the waves'
@@ -45,7 +45,6 @@ template <typename T>
 __device__ __forceinline__ gptr<T> gp(const void* p) { return (gptr<T>)(p); }
 
 constexpr int kBlk = 32;       // elements per packed block
-constexpr int kLanesRows = 2;  // up to this many rows: mnb_gemv_lanes_kernel
 
 // Elements 8 j .. 8 j + 7 of a packed block (its `BITS` words in registers), dequantised to f16 in the slot order
 // (e0, e4, e1, e5, e2, e6, e3, e7) of the slice: each 32-bit pair holds elements i and i + 4, which one shift and
@@ -168,7 +167,7 @@ __global__ __launch_bounds__(64 * kGW) void mnb_gemv_kernel(MnbArgs a) {
 // one column's packed row), dequantises them and multiplies them into the rows of a with v_dot2_f32_f16 (fp32
 // accumulation). The lanes' partial sums are added by DPP and permlane. Bound: round trips, in a kernel of a few us. Two
 // forms:
-//   two columns a wave (launch_lanes: below kLaneWide columns): the next blocks are loaded before the current ones are
+//   two columns a wave (below kLaneWide columns): the next blocks are loaded before the current ones are
 //     used, and the rows of a come through LDS, copied once per workgroup in whole lines while the first blocks are on
 //     their way: read directly, a lane's 64 bytes are a cache line of their own, twice the address cycles of two columns'
 //     weights. 2048 x 6144, weights rotating through eight matrices: 6.1 us with four columns a wave, 4.9 with two; two
@@ -339,7 +338,7 @@ __global__ __launch_bounds__(256) void mnb_gemv_wide_kernel(MnbArgs a) {
 // per k tile. Rows past M and columns past N load clamped rows and are not stored; a k tile past the last
 // block (K % 64 == 32) is zero in both operands. Tiles are numbered so that each XCD (workgroup id % 8) takes a
 // contiguous range of them, n fastest, sharing a rows in its L2.
-constexpr int kTN = 128, kTK = 64;
+constexpr int kTN = gemm::kTN, kTK = 64;
 typedef float f16v __attribute__((ext_vector_type(16)));
 // 16-byte chunk c (k 8 c .. 8 c + 7 of the tile) of row r sits in slot 8 r + (c ^ (r & 7)): the MFMA operand reads
 // of 32 rows at one chunk then fall in distinct banks without padding
@@ -601,7 +600,6 @@ void launch_fwht_log(_Float16* x, long blocks, float scale, hipStream_t s) {
   hipLaunchKernelGGL(fwht_kernel<LOG>, dim3((unsigned)((blocks + kPer - 1) / kPer)), dim3(kWG), 0, s, x, blocks, scale);
 }
 
-constexpr int kLaneWide = 4096;  // columns
 template <int BITS, int GROUP, bool ASYM, int MR>
 void launch_lanes(const MnbArgs& a, hipStream_t s) {
   if (a.N < kLaneWide)
@@ -633,7 +631,7 @@ template <int BITS, int GROUP, bool ASYM>
 hipError_t launch_gemm(const MnbArgs& a, hipStream_t s) {
   // 256-row tiles (8 waves) when they still give every CU a workgroup, else 128-row tiles (4 waves)
   const long ntn = (a.N + kTN - 1) / kTN, tiles256 = ntn * ((a.M + 255) / 256);
-  if (tiles256 >= 256)
+  if (gemm::tall(a.M, a.N))
     hipLaunchKernelGGL((mnb_gemm_kernel<BITS, GROUP, ASYM, 4>), dim3((unsigned)tiles256, a.split), dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL((mnb_gemm_kernel<BITS, GROUP, ASYM, 2>), dim3((unsigned)(ntn * ((a.M + 127) / 128)), a.split),
@@ -679,33 +677,11 @@ hipError_t mnb_check(const MnbArgs& a) {
   return hipSuccess;
 }
 
-MnbPath mnb_path(const MnbArgs& a) {
-  // One or two rows: the lanes kernel, from 4096 columns on the strip kernel (12288 / 8256 / 5120 x 2048: 5.9 / 5.3 / 4.7
-  // us against 6.8 / 6.0 / 5.0; 2048 x 2048 / 6144: 4.6 / 6.3 against 3.8 / 5.1). Operands that the DMAs of the strip and tile kernels cannot move (K % 64, alignment):
-  // the register-operand kernel up to 64 rows (10 - 28 us at 64 rows against 27 - 71 us for the GEMM), then the GEMM.
-  if (a.M <= kLanesRows) return a.N >= 4096 && mnb_strip_takes(a) ? kMnbStrip : kMnbGemv;
-  if (!mnb_strip_takes(a)) return a.M <= 64 ? kMnbGemv : kMnbGemm;
-  if (!mnb_tiles_takes(a)) return a.M <= 384 ? kMnbStrip : kMnbGemm;  // 2 and 3 bits
-  // 4 bits: up to 256 rows the strip kernel (a row's bits then depend on neither M nor the tiles), above it the one whose
-  // expected time is less
-  return a.M <= 256 || mnb_strip_us(a) < mnb_tiles_us(a) ? kMnbStrip : kMnbTiles;
-}
+MnbShape mnb_shape(const MnbArgs& a) { return MnbShape{a.M, a.N, a.K, a.bits, a.group, a.asym != 0, mnb_strip_takes(a)}; }
 
 hipError_t launch_mnb_gemv(const MnbArgs& a, hipStream_t s) {
   if (a.M < 1 || a.M > 64 || !a.a || !a.y) return hipErrorInvalidValue;
   return a.M <= kLanesRows ? dispatch_fmt<GemvLanesF>(a, s) : dispatch_fmt<GemvF>(a, s);
-}
-
-int mnb_gemm_split(int M, int N, int K) {
-  // Fewer output tiles than CUs leave CUs idle behind one long K loop each (about 0.85 us per 64-deep k tile):
-  // split K so that about 384 workgroups run, each over at least 4 k tiles, with at most 64 MiB of fp32 partials.
-  const long ntn = (N + kTN - 1) / kTN, tiles256 = ntn * ((M + 255) / 256);
-  const long tiles = tiles256 >= 256 ? tiles256 : ntn * ((M + 127) / 128);
-  const int nkt = (K / kBlk + 1) / 2;
-  if (tiles >= 256) return 1;
-  long sp = std::min<long>((384 + tiles - 1) / tiles, nkt / 4);
-  while (sp > 1 && sp * M * (long)N * 4 > (64L << 20)) sp--;
-  return (int)std::max<long>(sp, 1);
 }
 
 hipError_t launch_mnb_gemm(const MnbArgs& a, hipStream_t s) {

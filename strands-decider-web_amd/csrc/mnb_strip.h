@@ -191,11 +191,9 @@ hipError_t launch_one(const MnbArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Tile counts a format is built for: all for what the exporter writes (4 bits, groups of 32, symmetric), fewer shapes for
-// the others.
+// The tile counts of mnb_plan.h's built().
 template <int BITS, int GROUP, bool ASYM>
 constexpr bool kEveryTile = BITS == 4 && GROUP == 32 && !ASYM;
-bool every_tile(const MnbArgs& a) { return a.bits == 4 && a.group == 32 && !a.asym; }
 template <int BITS, int GROUP, bool ASYM>
 hipError_t launch_fmt(const MnbArgs& a, int mt, int nt, hipStream_t s) {
 #define HA_STRIP(MT, NT) \
@@ -211,31 +209,6 @@ hipError_t launch_fmt(const MnbArgs& a, int mt, int nt, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
-// The tile counts (mt, nt) of a shape. One workgroup fits a CU's LDS once to four times and its time grows with
-// mt + nt (rows of a and columns of W it reads), so: for each nt the fewest row tiles that give at most 256
-// workgroups a round, over the rounds that needs, and of those the least rounds x (mt + nt + 2). Measured choices
-// (M, N, K: mt x nt us, next best): 61, 2048, 6144: 2 x 1 8.0, 3 x 1 9.0; 61, 12288, 2048: 4 x 3 9.9, 2 x 3 10.4;
-// 128, 5120, 2048: 3 x 4 8.9, 4 x 3 9.1; 192, 8256, 2048: 4 x 4 18.0, 3 x 3 18.7.
-int pick_tiles(int M, int N, bool every, int* mt, int* nt) {
-  const int tm = (M + 15) / 16, tn = N / 16;
-  int best = 1 << 30;
-  *mt = *nt = 1;
-  for (int n = 1; n <= (every ? 4 : 3); n++) {
-    const int gx = (tn + n - 1) / n;
-    for (int rounds = 1; rounds <= 64; rounds++) {
-      const int rb = rounds * 256 / gx;
-      if (rb < 1) continue;
-      int m = (tm + rb - 1) / rb;
-      if (every) m = m == 7 ? 8 : m;
-      else m = m == 3 ? 4 : m;
-      if (m > (!every ? 4 : n == 4 ? 6 : 8)) continue;
-      const int cost = rounds * (m + n + 2);
-      if (cost < best) best = cost, *mt = m, *nt = n;
-    }
-  }
-  return best;
-}
-
 }  // namespace
 }  // namespace strip
 
@@ -246,16 +219,10 @@ bool mnb_strip_takes(const MnbArgs& a) {
          q % (a.bits == 4 ? 16 : 4) == 0 && sb % 4 == 0;
 }
 
-// rounds x (mt + nt + 2), in units of 0.35 us and 0.55 us for every 2048 of K (measured 0.8 to 1.1 of this)
-float mnb_strip_us(const MnbArgs& a) {
-  int mt, nt;
-  return (float)strip::pick_tiles(a.M, a.N, strip::every_tile(a), &mt, &nt) * (0.35f + 0.55f * a.K / 2048.0f);
-}
-
 hipError_t launch_mnb_strip(const MnbArgs& a, hipStream_t s) {
   if (a.M < 1 || !a.a || !a.y || !mnb_strip_takes(a)) return hipErrorInvalidValue;
   int mt = 0, nt = 0;
-  strip::pick_tiles(a.M, a.N, strip::every_tile(a), &mt, &nt);
+  strip::pick_tiles(a.M, a.N, strip::every_tile(mnb_shape(a)), &mt, &nt);
 #define HA_STRIP_CASE(B, G, S) \
   if (a.bits == B && a.group == G && a.asym == S) return strip::launch_fmt<B, G, S>(a, mt, nt, s);
   HA_STRIP_CASE(4, 32, false) HA_STRIP_CASE(4, 32, true) HA_STRIP_CASE(4, 64, false) HA_STRIP_CASE(4, 64, true)

@@ -183,7 +183,6 @@ hipError_t launch_shape(const MnbArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-enum Shape { k256x256, k128x256, k128x128 };
 template <int GROUP, bool ASYM>
 hipError_t launch_fmt(const MnbArgs& a, Shape sh, hipStream_t s) {
   if (sh == k256x256) return launch_shape<GROUP, ASYM, 4, 2, 2, 4, 2>(a, s);
@@ -195,36 +194,10 @@ hipError_t launch(const MnbArgs& a, Shape sh, hipStream_t s) {
   return a.asym ? launch_fmt<64, true>(a, sh, s) : launch_fmt<64, false>(a, sh, s);
 }
 
-// Columns [0, n1) by 256 x 256 tiles, [n1, n2) by `rest`, [n2, N) by the strip kernel; us: the time this is expected to take.
-struct Plan {
-  int n1, n2;
-  Shape rest;
-  float us;
-};
-// Measured, K = 2048: a round (at most one tile on each of the 256 CUs) takes 57, 29 and 20.5 us, plus a launch's own few;
-// full rounds end up at about 920 TFLOP/s whatever the shape (the clock falls: 256 tiles of 256 x 256 take 75 us, 160 59).
-Plan plan_tiles(int M, int N, int K) {
-  const int m256 = (M + 255) / 256, m128 = (M + 127) / 128, tail = N > 256 && N % 256 <= 64 ? N % 256 : 0, nt = N - tail;
-  auto rounds = [](long t) { return (float)((t + 255) / 256); };
-  Plan best{0, nt, k128x128, 1e30f};
-  for (int r = 0; r <= 64; r++) {
-    const int c1 = std::min(256 * r / m256, nt / 256);  // tile columns that fill r rounds
-    const int left = nt - 256 * c1;
-    const float t1 = c1 ? 57.0f * rounds((long)m256 * c1) : 0.0f;
-    const float tb = 29.0f * rounds((long)m128 * ((left + 255) / 256)), tc = 20.5f * rounds((long)m128 * ((left + 127) / 128));
-    const float busy = (float)M * nt * (2 * 2048 / 920e6f);
-    const float t = K / 2048.0f * std::max(t1 + std::min(tb, tc), busy) + (c1 ? 2.0f : 0.0f) + (left ? 3.0f : 0.0f) + (tail ? 5.0f : 0.0f);
-    if (t < best.us) best = {256 * c1, nt, tb <= tc ? k128x256 : k128x128, t};
-    if (c1 == nt / 256) break;
-  }
-  return best;
-}
-
 }  // namespace
 }  // namespace tiles
 
 bool mnb_tiles_takes(const MnbArgs& a) { return a.bits == 4 && mnb_strip_takes(a); }
-float mnb_tiles_us(const MnbArgs& a) { return tiles::plan_tiles(a.M, a.N, a.K).us; }
 
 hipError_t launch_mnb_tiles(const MnbArgs& a, hipStream_t s) {
   if (a.M < 1 || !a.a || !a.y || !mnb_tiles_takes(a)) return hipErrorInvalidValue;

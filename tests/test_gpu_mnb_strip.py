@@ -85,6 +85,33 @@ def test_many_rows(N, K, group, asym):
     w.close()
 
 
+@pytest.mark.parametrize("N,K,bits,group,asym,Ms", [
+    (33040, 128, 4, 32, True, [64, 129, 200]),   # beyond 12800 columns: strip, then tiles
+    (33040, 128, 4, 64, False, [129, 256]),
+    (151952, 64, 3, 32, False, [3, 64, 200, 384]),  # strip, then the GEMM
+    (151952, 64, 2, 32, True, [300, 385]),
+    (49168, 1088, 4, 32, False, [1, 2]),         # one row: four columns a wave; two rows: strip
+    (8208, 1088, 3, 32, True, [1, 2]), (8208, 1152, 2, 64, False, [1, 2]),
+    (8176, 1088, 4, 32, False, [1, 2]), (4112, 2080, 4, 32, True, [1, 2]), (8208, 2080, 3, 32, False, [1, 2])])
+def test_lines_of_the_rule(N, K, bits, group, asym, Ms):
+    # either side of the lines at which a call goes to another kernel (mnb_plan.h)
+    import torch
+    words, sc, bi = _weights(N, K, bits, group, asym, N + K + bits)
+    W = mo.dequant(words, sc, N, K, bits, group, asym, bi)
+    q, s, b = _dev(words), _dev(sc), _dev(bi) if asym else None
+    w = ha.MnbWeight(N, K, q, s, b, bits=bits, group=group, asym=asym)
+    a = ((np.random.default_rng(4).random((max(Ms), K)) - 0.5) * 2).astype(np.float16)
+    ad, ref = _dev(a), mo.matmul(a, W)
+    for M in Ms:
+        y = torch.full((M + 1, N), 7.0, dtype=torch.float16, device="cuda:0")
+        w.forward(M, ad, y)
+        torch.cuda.synchronize()
+        g = y.cpu().numpy()
+        assert mo.rel_err(g[:M].astype(np.float64), ref[:M]) < TOL, M
+        assert (g[M] == 7.0).all(), "row past M written (M = %d)" % M
+    w.close()
+
+
 @pytest.mark.parametrize("bits,off_q,off_s", [(4, 4, 0), (4, 0, 2), (3, 4, 2)])
 def test_unaligned_operands(bits, off_q, off_s):
     import torch
