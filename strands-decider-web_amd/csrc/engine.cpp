@@ -66,7 +66,7 @@ struct Layer {
   float* gnorm = nullptr;
   float* qn = nullptr;
   float* kn = nullptr;
-  float* S = nullptr;     // [B][H][DK][DV] state of a call that keeps no snapshot
+  float* S = nullptr;     // [B][H][DK][DV] state of a call that keeps no snapshot, or whose snapshot has no memory yet
   _Float16* K = nullptr;  // [B][HK][LT][HD]
   _Float16* V = nullptr;  // [B][HK][HD][LT] (transposed: positions contiguous)
 };
@@ -674,47 +674,60 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
     int rc;  // first call that forces the paired form on another shape
     if ((rc = grow(sc.duo_ring, e->need_duo_ring))) return rc;
   }
-  // the snapshot's memory first: the gated-delta layers write their state and raw rows straight into it. Every part is in
-  // one device block (256-byte aligned offsets), the engine's spare block when it is large enough; a new block is rounded up
-  // to 2 MiB so that the next snapshots of a growing context fit in it when it returns
+  // The snapshot's memory: every part in one device block (256-byte aligned offsets). Where the engine's spare block is large
+  // enough the gated-delta layers write their state straight into it. A new block (rounded up to 2 MiB so that the next
+  // snapshots of a growing context fit in it when it returns) is allocated after the layers' launches, so that the device
+  // does not wait for the allocation; the layers then write the engine's own state buffers, copied from there. (A call that
+  // is timed allocates first: the times hold no allocation.)
   SnapshotGuard kept{nullptr, st};
+  const size_t state_bytes = sizeof(float) * B * c.H * c.DK * c.DV, kv_bytes = (size_t)end * c.HD * sizeof(_Float16) * B * c.HK;
+  size_t tail_bytes = 0, total = 0;
+  auto aligned = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  auto place = [&](void* block, size_t bytes) {
+    ha_snapshot* s = kept.s;
+    s->block = block; s->block_bytes = bytes;
+    size_t off = 0;
+    auto take = [&](size_t b) { void* q = static_cast<char*>(block) + off; off += aligned(b); return q; };
+    for (int i = 0; i < c.n_layers; i++) {
+      ha_snapshot::Part& p = s->layers[i];
+      if (e->layers[i].kind == HA_LINEAR_ATTENTION) {
+        p.S = static_cast<float*>(take(state_bytes));
+        p.tail = take(tail_bytes);
+      } else if (e->layers[i].kind == HA_FULL_ATTENTION) {
+        p.K = static_cast<_Float16*>(take(kv_bytes));
+        p.V = static_cast<_Float16*>(take(kv_bytes));
+      }
+    }
+  };
+  auto allocate = [&]() {
+    const size_t bytes = (total + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+    char* block = nullptr;
+    int rc = dalloc(&block, bytes);
+    if (rc == HA_OK) place(block, bytes);
+    return rc;
+  };
   if (keep) {
     ha_snapshot* s = kept.s = new ha_snapshot();
     s->owner = e; s->owner_id = e->id; s->uid = ++g_snap_uid; s->P = end; s->s0 = e->any_linear ? s1 : end;
     s->tail_rows = s->P - (s->s0 - (kKC - 1));
     s->layers.resize(c.n_layers);
-    auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t state = sizeof(float) * B * c.H * c.DK * c.DV, tail = dtype_size(c.lin_dtype) * c.lin_stride * B * s->tail_rows;
-    const size_t kv = (size_t)end * c.HD * sizeof(_Float16) * B * c.HK;
-    size_t total = 0;
+    tail_bytes = dtype_size(c.lin_dtype) * c.lin_stride * B * s->tail_rows;
     for (const Layer& l : e->layers)
-      total += l.kind == HA_LINEAR_ATTENTION ? al(state) + al(tail) : l.kind == HA_FULL_ATTENTION ? 2 * al(kv) : 0;
+      total += l.kind == HA_LINEAR_ATTENTION ? aligned(state_bytes) + aligned(tail_bytes) : l.kind == HA_FULL_ATTENTION ? 2 * aligned(kv_bytes) : 0;
+    void* spare = nullptr;
+    size_t spare_bytes = 0;
     {
       std::lock_guard<std::mutex> lock(g_live_mu);
       if (e->spare && e->spare_bytes >= total) {
-        s->block = e->spare; s->block_bytes = e->spare_bytes;
-        e->spare = nullptr; e->spare_bytes = 0;
+        std::swap(spare, e->spare);
+        std::swap(spare_bytes, e->spare_bytes);
       }
     }
-    if (!s->block) {
-      const size_t bytes = (total + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
-      int rc = dalloc(reinterpret_cast<char**>(&s->block), bytes);
-      if (rc) return rc;
-      s->block_bytes = bytes;
-    }
-    size_t off = 0;
-    auto take = [&](size_t b) { void* q = static_cast<char*>(s->block) + off; off += al(b); return q; };
-    for (int i = 0; i < c.n_layers; i++) {
-      ha_snapshot::Part& p = s->layers[i];
-      if (e->layers[i].kind == HA_LINEAR_ATTENTION) {
-        p.S = static_cast<float*>(take(state));
-        p.tail = take(tail);
-      } else if (e->layers[i].kind == HA_FULL_ATTENTION) {
-        p.K = static_cast<_Float16*>(take(kv));
-        p.V = static_cast<_Float16*>(take(kv));
-      }
-    }
+    if (spare) place(spare, spare_bytes);
+    else if (timing)
+      if (int rc = allocate()) return rc;
   }
+  const bool late = keep && !kept.s->block;  // the block comes after the launches
   // raw-row tails of a kept snapshot: the copy reads only the call's input rows and the resumed tail, so the layers'
   // copies are gathered into one launch after the mixers (per layer when per-layer times are asked for, so that each
   // layer's time includes its own copy). A call that keeps no snapshot copies nothing: only a snapshot's rows are read
@@ -724,9 +737,14 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
   t.P = P; t.L = L; t.s0 = s0; t.KC = kKC; t.tail_cap_in = resume ? resume->tail_rows : kKC - 1;
   t.tail_cap_out = keep ? kept.s->tail_rows : 0; t.dst_first = s1 - (kKC - 1); t.dtype = c.lin_dtype == HA_F16 ? 1 : 0;
   auto flush_tails = [&]() {
-    const hipError_t he = ha::launch_tail_update(t, st);
+    const hipError_t he = t.n > 0 ? ha::launch_tail_update(t, st) : hipSuccess;
     t.n = 0;
     return he;
+  };
+  auto add_tail = [&](int i) {
+    t.in[t.n] = layer_in[i]; t.tail[t.n] = resume ? resume->layers[i].tail : sc.zeros.p; t.tail_out[t.n] = kept.s->layers[i].tail;
+    t.n++;
+    return t.n == ha::kTailLayers ? flush_tails() : hipSuccess;
   };
   if (timing) HA_HIP(hipEventRecord(e->ev[0], st));
   for (int i = 0; i < c.n_layers; i++) {
@@ -740,7 +758,7 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       a.tail_cap = resume ? resume->tail_rows : kKC - 1;
       a.dtype = c.lin_dtype == HA_F16 ? 1 : 0;
       a.in = layer_in[i]; a.out = layer_out[i];
-      a.S_in = resume ? resume->layers[i].S : nullptr; a.S_out = keep ? kept.s->layers[i].S : l.S;
+      a.S_in = resume ? resume->layers[i].S : nullptr; a.S_out = keep && !late ? kept.s->layers[i].S : l.S;
       a.keep_state = keep != nullptr;
       a.conv_w = l.conv; a.negA = l.negA; a.dtb = l.dtb; a.gnorm = c.lin_gnorm ? l.gnorm : nullptr;
       a.img = sc.img.p; a.img_chunks = e->img_chunks;
@@ -766,11 +784,9 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       }
       if (he != hipSuccess) return fail(HA_ERR_DEVICE, "layer " + std::to_string(i) + " gated-delta launch: " + hipGetErrorString(he));
       if (per_layer) HA_HIP(hipEventRecord(e->mev[i], st));
-      if (keep) {
-        t.in[t.n] = a.in; t.tail[t.n] = a.tail; t.tail_out[t.n] = kept.s->layers[i].tail; t.n++;
-      }
-      if (t.n > 0 && (per_layer || t.n == ha::kTailLayers)) {
-        he = flush_tails();
+      if (keep && !late) {
+        he = add_tail(i);
+        if (he == hipSuccess && per_layer) he = flush_tails();
         if (he != hipSuccess) return fail(HA_ERR_DEVICE, "layer " + std::to_string(i) + " tail update: " + hipGetErrorString(he));
       }
     } else if (l.kind == HA_FULL_ATTENTION) {
@@ -805,10 +821,16 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       HA_HIP(hipEventRecord(e->mev[i], st));
     }
   }
-  if (t.n > 0) {
-    const hipError_t he = flush_tails();
-    if (he != hipSuccess) return fail(HA_ERR_DEVICE, std::string("tail update: ") + hipGetErrorString(he));
+  if (late) {
+    if (int rc = allocate()) return rc;
+    for (int i = 0; i < c.n_layers; i++) {
+      if (e->layers[i].kind != HA_LINEAR_ATTENTION) continue;
+      HA_HIP(hipMemcpyAsync(kept.s->layers[i].S, e->layers[i].S, state_bytes, hipMemcpyDeviceToDevice, st));
+      HA_HIP(add_tail(i));
+    }
   }
+  if (const hipError_t he = flush_tails(); he != hipSuccess)
+    return fail(HA_ERR_DEVICE, std::string("tail update: ") + hipGetErrorString(he));
   if (per_layer) HA_HIP(hipEventRecord(e->lev[c.n_layers], st));
   if (timing) HA_HIP(hipEventRecord(e->ev[1], st));
 
