@@ -369,8 +369,8 @@ __global__ __launch_bounds__(64 * kWaves) void gqa_attn_kernel(GqaArgs a, int pe
         const float n1 = x1[e] * inv * (e < 4 ? w10[e] : w11[e - 4]), n2 = x2[e] * inv * (e < 4 ? w20[e] : w21[e - 4]);
         const f4 c = rz[ks][e >> 1];
         const float cs = c[2 * (e & 1)], sn = c[2 * (e & 1) + 1];
-        r1[e] = (_Float16)(n1 * cs - n2 * sn);
-        r2[e] = (_Float16)(n2 * cs + n1 * sn);
+        r1[e] = fma_f16(n1, cs, -(n2 * sn));
+        r2[e] = fma_f16(n2, cs, n1 * sn);
       }
       qreg[ks] = r1 * scale;
       qreg[ks + 2] = r2 * scale;

@@ -95,11 +95,21 @@ __device__ __forceinline__ float wave_sum64(float v) {
   return sum_halves(v);
 }
 
+// The general and the short-call kernels have to give the same bits, so every rounding that the compiler could choose is written
+// out: which of two products a sum fuses (it has chosen differently in two kernels of the same source), and whether an f16
+// result is rounded to f32 first.
+// f16(a b + c), one rounding.
+__device__ __forceinline__ _Float16 fma_f16(float a, float b, float c) {
+  unsigned r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return __builtin_bit_cast(_Float16, (unsigned short)r);
+}
+
 // Key row of one position from a lane's 4 raw dims x (dims 4 lane .. + 3 of the wave's 64 lanes): RMSNorm, gain kw and
 // rotate-half RoPE on dims [0, 64) (dim i < 32 pairs with i + 32, held by lane l ^ 8); cs0, cs1: the lane's four
 // (cos, sin) pairs, used by lanes < 16.
 __device__ __forceinline__ f4 key_row(const f4& x, const f4& kw, const f4& cs0, const f4& cs1, int lane) {
-  const float ss = wave_sum64((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]));
+  const float ss = wave_sum64(__builtin_fmaf(x[0], x[0], x[1] * x[1]) + __builtin_fmaf(x[2], x[2], x[3] * x[3]));
   const float inv = rsqrtf(ss / kHD + 1e-6f);
   f4 k = x * inv * kw;
   f4 pk;
@@ -108,7 +118,7 @@ __device__ __forceinline__ f4 key_row(const f4& x, const f4& kw, const f4& cs0, 
   if (lane < 16) {
     const float cs[4] = {cs0[0], cs0[2], cs1[0], cs1[2]}, sn[4] = {cs0[1], cs0[3], cs1[1], cs1[3]};
 #pragma unroll
-    for (int c = 0; c < 4; c++) k[c] = lane < 8 ? k[c] * cs[c] - pk[c] * sn[c] : k[c] * cs[c] + pk[c] * sn[c];
+    for (int c = 0; c < 4; c++) k[c] = __builtin_fmaf(k[c], cs[c], lane < 8 ? -(pk[c] * sn[c]) : pk[c] * sn[c]);
   }
   return k;
 }

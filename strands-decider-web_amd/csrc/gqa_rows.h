@@ -66,14 +66,6 @@ __device__ __forceinline__ int group_tiles(const GqaArgs& a, int grp) {
   return min(a.P + grp * kG + kG - 1, a.P + a.L - 1) / kBK + 1;
 }
 
-// f16(a b + c) with the one instruction gqa_attn_kernel's code rounds a rotated pair with (written out: left to itself the
-// compiler may round to f32 first, or fuse the other product, and a bit in a thousand rows would differ)
-__device__ __forceinline__ _Float16 fma_f16(float a, float b, float c) {
-  unsigned r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return __builtin_bit_cast(_Float16, (unsigned short)r);
-}
-
 // Q as the B operand of S^T = K Q^T: qreg[ks] = q[row c32 of the group][16 ks + 8 half .. + 7] after RMSNorm, gain, RoPE
 // and the scale 2^-4, with gqa_attn_kernel's roundings and order of sums. A row past the call's end repeats the last one.
 // load() issues an f16 row's loads (an f32 row is read in pieces later).
