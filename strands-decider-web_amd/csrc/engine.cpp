@@ -25,6 +25,7 @@
 #include <unordered_set>
 #include <vector>
 
+#include "gqa_plan.h"
 #include "ha.h"
 #include "ha_kernels.h"
 
@@ -111,6 +112,16 @@ int grow(Scratch::Buf& b, size_t bytes, bool zero = true) {
   if (b.p) (void)hipFree(b.p);
   b.p = p;
   b.bytes = bytes;
+  return HA_OK;
+}
+
+// The short-call attention scratch and its marks. Without the memory for them such calls are served by the general kernel,
+// which computes the same bits.
+int grow_rows(Scratch& s, size_t rows, size_t marks) {
+  int rc = grow(s.gqa_rows, rows, false);
+  if (rc == HA_OK) rc = grow(s.gqa_marks, marks);
+  if (rc != HA_ERR_NOMEM) return rc;
+  (void)hipGetLastError();  // dealt with
   return HA_OK;
 }
 
@@ -486,8 +497,7 @@ int ha_create(const ha_config* cfg, int device, ha_engine** out) {
     }
     e->need_gqa_rows = ha::gqa_rows_bytes((int)B * c.HK, c.max_ctx);
     e->need_gqa_marks = ha::gqa_rows_marks((int)B * c.HK, c.max_ctx) * sizeof(unsigned);
-    if ((rc = grow(e->scratch->gqa_rows, e->need_gqa_rows, false)) || (rc = grow(e->scratch->gqa_marks, e->need_gqa_marks)))
-      return bail(rc);
+    if ((rc = grow_rows(*e->scratch, e->need_gqa_rows, e->need_gqa_marks))) return bail(rc);
     if (hipMemcpy(e->rope, rope.data(), rope.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(HA_ERR_DEVICE, "hipMemcpy rope failed"));
   }
@@ -522,8 +532,8 @@ int ha_set_stream(ha_engine* e, void* stream) {
     int rc;
     if ((rc = grow(s->zeros, e->need_zeros)) || (rc = grow(s->seq_raw, e->need_seq_raw)) ||
         (rc = grow(s->seq_cnt, e->need_seq_cnt)) || (rc = grow(s->sync_flags, e->need_sync_flags)) ||
-        (rc = grow(s->gqa_part, e->need_gqa)) || (rc = grow(s->gqa_rows, e->need_gqa_rows, false)) ||
-        (rc = grow(s->gqa_marks, e->need_gqa_marks)) || (rc = grow(s->img, split_by_shape(c) ? e->need_img : 0)) ||
+        (rc = grow(s->gqa_part, e->need_gqa)) || (rc = grow_rows(*s, e->need_gqa_rows, e->need_gqa_marks)) ||
+        (rc = grow(s->img, split_by_shape(c) ? e->need_img : 0)) ||
         (rc = grow(s->duo_ring, paired_by_shape(c) ? e->need_duo_ring : 0)))
       return rc;
     std::lock_guard<std::mutex> lock(g_live_mu);
@@ -551,7 +561,7 @@ int ha_share_scratch(ha_engine* e, ha_engine* holder) {
   if ((rc = grow(to.zeros, e->need_zeros)) || (rc = grow(to.img, from.img.bytes ? e->need_img : 0)) ||
       (rc = grow(to.seq_raw, e->need_seq_raw)) ||
       (rc = grow(to.seq_cnt, e->need_seq_cnt)) || (rc = grow(to.gqa_part, e->need_gqa)) ||
-      (rc = grow(to.gqa_rows, e->need_gqa_rows, false)) || (rc = grow(to.gqa_marks, e->need_gqa_marks)) ||
+      (rc = grow_rows(to, e->need_gqa_rows, e->need_gqa_marks)) ||
       (rc = grow(to.duo_ring, from.duo_ring.bytes ? e->need_duo_ring : 0)) ||
       (rc = grow(to.sync_flags, e->need_sync_flags)))
     return rc;
@@ -796,7 +806,8 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       a.in = layer_in[i]; a.out = layer_out[i]; a.qw = l.qn; a.kw = l.kn; a.rope = e->rope;
       a.K = l.K; a.V = l.V;
       a.split = e->gqa_split; a.part_slots = e->gqa_part_slots; a.part = static_cast<float*>(sc.gqa_part.p);
-      a.rows = sc.gqa_rows.p; a.row_marks = static_cast<unsigned*>(sc.gqa_marks.p);
+      a.rows = sc.gqa_rows.p; a.rows_bytes = sc.gqa_rows.bytes;
+      a.row_marks = static_cast<unsigned*>(sc.gqa_marks.p); a.marks_bytes = sc.gqa_marks.bytes;
       const bool rows = ha::gqa_rows_takes(a);
       if (a.split > 0 && !rows) {
         // a fresh mark per launch; if the counter wraps, the marks (and partials) are cleared first

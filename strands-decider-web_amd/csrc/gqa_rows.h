@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "gqa_common.h"
+#include "gqa_plan.h"
 #include "ha_kernels.h"
 #include "lds_dma.h"
 
@@ -31,37 +32,14 @@ namespace ha {
 namespace gqa_rows {
 namespace {
 
-constexpr int kG = 32;           // query rows of a group
 constexpr int kSW = 8;           // waves of a scores workgroup: query head w & 3, 32-key half w >> 2 of the tile
-constexpr int kMaxPieces = 8;    // waves of a values workgroup with split key ranges
-constexpr int kPUnit = 2048;     // bytes of P of one 32-key half: [k-step][lane] 16 bytes
-constexpr int kSUnit = 32 * 8;   // bytes of a half's row statistics: [row] (alpha, sum)
-constexpr int kMUnit = 32 * 4;   // bytes of a half's row maxima, and of its reference maxima
-
-// Scratch of a call: per chain unit u = ((pair * ngrp + group) * 4 + head) * nh + half all P, then all statistics, all
-// maxima, all reference maxima. The marks [pair][group][tile] are a buffer of their own, so that no other data ever lies where a mark is
-// looked for. They are zero between calls: a scores workgroup sets its own, the values kernel clears them again, so a
-// launch that a graph replays waits for its own marks and not for those of the replay before.
-constexpr unsigned kMark = 1;
-struct RowsLayout {
-  int ngrp, nt, nh;  // query groups, tiles of the longest group, halves
-  unsigned units;    // chain units in all
-};
-__host__ __device__ inline RowsLayout rows_layout(const GqaArgs& a) {
-  RowsLayout r;
-  r.ngrp = (a.L + kG - 1) / kG;
-  r.nt = (a.P + a.L - 1) / kBK + 1;
-  r.nh = 2 * r.nt;
-  r.units = (unsigned)(a.B * a.HK * r.ngrp * 4) * (unsigned)r.nh;
-  return r;
-}
-constexpr size_t kUnitBytes = kPUnit + kSUnit + 2 * kMUnit;
+static_assert(kTile == kBK, "the tiles of gqa_attn_kernel");
 typedef float f2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ unsigned unit_of(const RowsLayout& r, int pair, int grp, int head, int half) {
   return (((unsigned)pair * r.ngrp + grp) * 4 + head) * r.nh + half;
 }
-// the last position group grp of the call sees
+// key tiles that query group grp of the call sees
 __device__ __forceinline__ int group_tiles(const GqaArgs& a, int grp) {
   return min(a.P + grp * kG + kG - 1, a.P + a.L - 1) / kBK + 1;
 }
@@ -587,31 +565,8 @@ hipError_t launch(const GqaArgs& a, hipStream_t s) {
 }  // namespace
 }  // namespace gqa_rows
 
-// The longest call taken, rows a sequence. gqa_attn_kernel has one workgroup per 64 rows and pair (pieces of 8 tiles in
-// engines of one or two pairs), so it catches up as rows and pairs fill the chip; the lines lie where it does. Measured at
-// 0 to 3000 cached keys, its time over this one's: 2 pairs 1.02 .. 2.6 at up to 256 rows (0.99 .. 1.02 at 400); 4 to 16
-// pairs 1.02 .. 3.1 at up to 128; 32 pairs 1.00 .. 1.5 at up to 64 but 0.5 .. 1.0 at 128; 64 pairs 0.5 .. 1.1 at any.
-int gqa_rows_max(int pairs) { return pairs <= 2 ? 256 : pairs <= 16 ? 128 : pairs <= 32 ? 64 : 0; }
-
-size_t gqa_rows_marks(int pairs, int max_ctx) {
-  return (size_t)pairs * ((gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG) * ((max_ctx + kBK - 1) / kBK);
-}
-size_t gqa_rows_bytes(int pairs, int max_ctx) {
-  const size_t groups = (gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG, halves = 2 * (size_t)((max_ctx + kBK - 1) / kBK);
-  return pairs * groups * 4 * halves * gqa_rows::kUnitBytes;
-}
-
-// (HD, RD, heads per pair, LT: as launch_gqa checks them)
-bool gqa_rows_takes(const GqaArgs& a) {
-  return a.rows && a.row_marks && a.L <= gqa_rows_max(a.B * a.HK) && a.HD == kHD && a.RD == 64 && a.HQ == 4 * a.HK &&
-         a.LT % kBK == 0;
-}
-
 hipError_t launch_gqa_rows(const GqaArgs& a, hipStream_t s) {
-  if (!gqa_rows_takes(a) || a.P + a.L > a.LT) return hipErrorInvalidValue;
-  if (a.split > 0 && (a.LT / kBK + a.split - 1) / a.split > gqa_rows::kMaxPieces) return hipErrorInvalidValue;
-  // maxima are addressed by 32-bit byte offsets
-  if ((size_t)gqa_rows::rows_layout(a).units * gqa_rows::kMUnit > 0x7fffffff) return hipErrorInvalidValue;
+  if (!gqa_rows_takes(a)) return hipErrorInvalidValue;
   return a.dtype == 0 ? gqa_rows::launch<float>(a, s) : gqa_rows::launch<_Float16>(a, s);
 }
 

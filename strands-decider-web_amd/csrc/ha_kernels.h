@@ -82,20 +82,16 @@ struct GqaArgs {
   float* part;               // [slots][4][64][HD] unnormalised O, then [slots][4][64][2] (reference max, sum), then
                              // [slots] u32 epoch marks
   unsigned epoch;            // split key ranges: this launch's mark, >= 1 and different from every earlier launch's on `part`
-  void* rows;                // short calls: scratch of gqa_rows_bytes(), or nullptr
-  unsigned* row_marks;       // short calls: gqa_rows_marks() marks, zero between calls
+  void* rows;                // short calls: scratch, or nullptr
+  unsigned* row_marks;       // short calls: marks, zero between calls
+  size_t rows_bytes, marks_bytes;
   WaitCheck wait;            // the merge workgroups' bounded wait for their pieces
 };
 
 // Slots of partial results the split GQA path needs for any call on a context of at most max_ctx positions.
 size_t gqa_part_slots(int pairs, int max_ctx, int split);
 size_t gqa_part_slot_bytes();
-// Short calls (at most gqa_rows_max(pairs) rows a sequence): every key tile on a workgroup of its own, then every slice of
-// output dims. Needs scratch for any such call on a context of at most max_ctx positions.
-int gqa_rows_max(int pairs);
-size_t gqa_rows_bytes(int pairs, int max_ctx);
-size_t gqa_rows_marks(int pairs, int max_ctx);
-bool gqa_rows_takes(const GqaArgs& a);
+// Short calls (gqa_plan.h): every key tile on a workgroup of its own, then every slice of output dims.
 hipError_t launch_gqa_rows(const GqaArgs& a, hipStream_t s);
 
 // Copy the raw rows [dst_first, P + L) (dst_first >= s0 - (KC-1)) of every sequence from (tail, in) into

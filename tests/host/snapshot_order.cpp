@@ -2,14 +2,6 @@
 // the call's state and raw rows.
 #include "fake_hip.h"
 
-// no short calls here
-namespace ha {
-int gqa_rows_max(int) { return 0; }
-size_t gqa_rows_bytes(int, int) { return 64; }
-size_t gqa_rows_marks(int, int) { return 64; }
-bool gqa_rows_takes(const GqaArgs&) { return false; }
-}  // namespace ha
-
 int main() {
   const unsigned char kinds[4] = {HA_LINEAR_ATTENTION, HA_ADAPTER, HA_LINEAR_ATTENTION, HA_FULL_ATTENTION};
   const ha_config c = config(kinds, 4, 1, 512);
@@ -31,7 +23,7 @@ int main() {
       const bool fresh = where("malloc") >= 0;
       CHECK(fresh == (round == 0 || (round == 2 && !timed)));
       if (fresh && !timed) {  // behind the last mixer, in front of what needs the memory
-        CHECK(where("malloc") > where("gqa") && where("malloc") < where("tails") && where("malloc") < where("copy2d"));
+        CHECK(where("malloc") > where("gqa_rows") && where("gqa_rows") >= 0 && where("malloc") < where("tails") && where("malloc") < where("copy2d"));
         CHECK(where("launch", where("malloc")) < 0);
       }
       if (fresh && timed) CHECK(where("malloc") < where("event"));  // the times hold no allocation

@@ -22,7 +22,7 @@ def engine(tmp_path_factory):
     return d, flags
 
 
-@pytest.mark.parametrize("name", ["snapshot_order"])
+@pytest.mark.parametrize("name", ["snapshot_order", "gqa_scratch"])
 def test_host(engine, name):
     d, flags = engine
     src = os.path.join(ROOT, "tests", "host", name + ".cpp")
