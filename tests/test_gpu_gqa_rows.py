@@ -14,13 +14,15 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("B,P,steps", [
     (1, 0, [1, 31, 32, 33]), (1, 63, [1, 1, 64, 65, 256]), (1, 509, [3, 129, 255]), (1, 1983, [64, 1]),
-    (2, 0, [128, 1]), (3, 191, [1, 33, 96, 128]), (8, 60, [5, 64]), (16, 100, [32, 64, 7])])
+    (2, 0, [128, 1]), (3, 191, [1, 33, 96, 128]), (8, 60, [5, 64]), (16, 100, [32, 64, 7]),
+    (2, 2030, [17, 1, 33, 128]), (3, 2900, [1, 100])])
 def test_rows_equal_a_long_forward(B, P, steps, f32):
-    # the long forward has more rows than any short call: the general kernel
+    # the long forward has more rows than any short call: the general kernel; contexts of more than 2048 positions have more
+    # tiles than the values kernel holds in LDS at a time
     T = max(P + sum(steps), 300)
     x = synth.gqa_rows(T, B, seed=31)
     x = x.astype(np.float32) if f32 else x
-    r = Runner(["full_attention"], batch=B, max_ctx=2048, **({"full_dtype": ha.F32} if f32 else {}))
+    r = Runner(["full_attention"], batch=B, max_ctx=2048 if T <= 2048 else 4096, **({"full_dtype": ha.F32} if f32 else {}))
     r.set_params(0, synth.gqa_params(seed=31, noise=0.1))
     (full,), whole = r.forward([x], keep=True)
     s, a = None, P

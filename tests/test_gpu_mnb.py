@@ -1,8 +1,9 @@
 """GPU parity of the MatMulNBits projections (ha_mnb_forward through the C ABI) against the fp64 oracle: the model's
-projection shapes (web/public/gemmbench/portable.js:18) across the three implementations (M <= 2: lanes kernel;
-M <= 64: packed-weight MFMA GEMV; larger M: the tiled GEMM that dequantises weight tiles into LDS, with its K range
-split over workgroups when there are few output tiles), every weight format of gemmbench/kernels.js:1-14, ragged
-tile edges, the exporter's own int4 quantiser, and the FWHT input rotation."""
+projection shapes (web/public/gemmbench/portable.js:18) across the implementations (one or two rows: lanes or strip
+kernel; few rows: strip kernel; many: tile kernel; K or alignment that these cannot move, and 2 and 3 bits with many
+rows: the packed-weight MFMA GEMV up to 64 rows, above that the tiled GEMM that dequantises weight tiles into LDS, with
+its K range split over workgroups when there are few output tiles), every weight format of gemmbench/kernels.js:1-14,
+ragged tile edges, the exporter's own int4 quantiser, and the FWHT input rotation."""
 import os
 import sys
 
@@ -80,15 +81,14 @@ def test_exporter_quantised_weights():
 
 @pytest.mark.parametrize("N,K", [(2048, 2048), (4096, 2048)])
 def test_implementations_agree_at_the_boundaries(N, K):
-    # the first rows computed with M = 2 (lanes kernel), 3 and 64 (MFMA GEMV), 65 and 200 (tiled GEMM, K split
-    # over workgroups)
+    # the first rows computed with M = 2 (lanes kernel), 3 to 200 (strip kernel) and 2000 (tile kernel)
     import torch
     words, sc, _ = _weights(N, K, seed=9)
     dev = "cuda:0"
     w = ha.MnbWeight(N, K, torch.from_numpy(words.view(np.int32)).to(dev), torch.from_numpy(sc).to(dev), None)
-    a = torch.from_numpy(((np.random.default_rng(2).random((200, K)) - 0.5) * 2).astype(np.float16)).to(dev)
+    a = torch.from_numpy(((np.random.default_rng(2).random((2000, K)) - 0.5) * 2).astype(np.float16)).to(dev)
     ys = {}
-    for M in (2, 3, 64, 65, 200):
+    for M in (2, 3, 64, 65, 200, 2000):
         ys[M] = torch.empty(M, N, dtype=torch.float16, device=dev)
         w.forward(M, a, ys[M])
     torch.cuda.synchronize()
@@ -102,8 +102,15 @@ def test_implementations_agree_at_the_boundaries(N, K):
 
 @pytest.mark.parametrize("N,K,Ms,bits,group,asym", [
     (1040, 2080, [49, 130, 257], 4, 32, False),   # N % 128 = 16, K % 64 = 32, M % 128 != 0
-    (2064, 2048, [200], 3, 64, True),
+    (1040, 2080, [65, 300], 4, 32, True),
+    (1040, 2112, [17, 70, 300], 4, 64, True),     # groups of 64, K % 128 = 64
+    (1040, 2112, [200], 4, 64, False),
+    (2064, 2048, [200, 400], 3, 64, True),        # strip, GEMM with K split
+    (528, 1088, [385], 2, 32, True),
+    (8208, 96, [1000], 4, 32, True),              # 256-row GEMM tiles
+    (8208, 128, [1000], 2, 64, False), (8208, 128, [1000], 3, 32, True),
     (16, 64, [1, 3, 50, 129], 2, 32, True),       # one 16-column tile, two blocks
+    (16, 96, [1, 3, 50, 129], 2, 32, True),
 ])
 def test_gemm_edges(N, K, Ms, bits, group, asym):
     words, sc, bi = _weights(N, K, bits, group, asym, seed=N + K)
@@ -113,9 +120,9 @@ def test_gemm_edges(N, K, Ms, bits, group, asym):
 
 
 def test_gemm_large_m_sampled_rows():
-    # one call with every row of a B = 8, T = 2048 prefill (M = 16384) on the largest input projection; a sample of
-    # rows against the oracle (the full fp64 product is too slow on the CPU); rows 0..2047 bit-identical to an
-    # M = 2048 call (same tiles, no K split), rows 0..63 within the bar of the M = 64 GEMV
+    # one call with every row of a B = 8, T = 2048 prefill (M = 16384) on the largest input projection (the tile kernel); a
+    # sample of rows against the oracle (the full fp64 product is too slow on the CPU); rows 0..2047 bit-identical to an
+    # M = 2048 call (its order of sums is the same for every tile shape), rows 0..63 within the bar of an M = 64 call (strip)
     import torch
     N, K, M = 8256, 2048, 16384
     words, sc, _ = _weights(N, K, seed=77)
@@ -125,7 +132,7 @@ def test_gemm_large_m_sampled_rows():
     y = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
     y64 = torch.empty(64, N, dtype=torch.float16, device=dev)
     y2k = torch.empty(2048, N, dtype=torch.float16, device=dev)
-    print("gemm M=%d N=%d K=%d" % (M, N, K), flush=True)
+    print("M=%d N=%d K=%d" % (M, N, K), flush=True)
     w.forward(M, a, y)
     w.forward(64, a, y64)
     w.forward(2048, a, y2k)

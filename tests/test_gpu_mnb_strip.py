@@ -112,19 +112,25 @@ def test_lines_of_the_rule(N, K, bits, group, asym, Ms):
     w.close()
 
 
-@pytest.mark.parametrize("bits,off_q,off_s", [(4, 4, 0), (4, 0, 2), (3, 4, 2)])
-def test_unaligned_operands(bits, off_q, off_s):
+@pytest.mark.parametrize("bits,off_q,off_s,group,asym,M", [
+    (4, 4, 0, 32, False, 40), (4, 0, 2, 32, False, 40), (3, 4, 2, 32, False, 40), (4, 4, 2, 32, True, 1), (4, 4, 0, 32, True, 200),
+    (4, 4, 2, 64, False, 200), (4, 0, 2, 64, True, 500), (2, 4, 2, 64, True, 200)])
+def test_unaligned_operands(bits, off_q, off_s, group, asym, M):
     import torch
-    N, K, M = 272, 256, 40
-    words, sc, _ = _weights(N, K, bits, 32, False, bits + off_q)
+    N, K = 272, 256
+    words, sc, bi = _weights(N, K, bits, group, asym, bits + off_q)
     qb = torch.zeros(words.size + 4, dtype=torch.int32, device="cuda:0")
     sb = torch.zeros(sc.size + 4, dtype=torch.float16, device="cuda:0")
     qb[off_q // 4:off_q // 4 + words.size] = _dev(words).reshape(-1)
     sb[off_s // 2:off_s // 2 + sc.size] = _dev(sc).reshape(-1)
-    w = ha.MnbWeight(N, K, qb.data_ptr() + off_q, sb.data_ptr() + off_s, None, bits=bits)
+    bb = torch.zeros(sc.size + 4, dtype=torch.float16, device="cuda:0")
+    if asym:
+        bb[off_s // 2:off_s // 2 + sc.size] = _dev(bi).reshape(-1)
+    w = ha.MnbWeight(N, K, qb.data_ptr() + off_q, sb.data_ptr() + off_s, bb.data_ptr() + off_s if asym else None, bits=bits,
+                     group=group, asym=asym)
     a = ((np.random.default_rng(2).random((M, K)) - 0.5) * 2).astype(np.float16)
     y = torch.empty(M, N, dtype=torch.float16, device="cuda:0")
     w.forward(M, _dev(a), y)
     torch.cuda.synchronize()
-    assert mo.rel_err(y.double().cpu().numpy(), mo.matmul(a, mo.dequant(words, sc, N, K, bits))) < TOL
+    assert mo.rel_err(y.double().cpu().numpy(), mo.matmul(a, mo.dequant(words, sc, N, K, bits, group, asym, bi))) < TOL
     w.close()

@@ -107,6 +107,20 @@ def test_paths(plan):
                 assert (strip if path == STRIP else gemm) <= 1.05 * min(strip, gemm), (s, r)
 
 
+def test_shapes_of_the_no_allocation_test(plan):
+    # the calls of test_zz_no_alloc.py whose partial products go to the fixed scratch: all but the last two shapes'
+    from test_zz_no_alloc import SHAPES
+    for n, (N, K, Ms, bits) in enumerate(SHAPES):
+        for r, M in zip(plan([(M, N, K, bits, 32, 0, K % 64 == 0) for M in Ms]), Ms):
+            path, split = r[0], r[8]
+            if n < 4:
+                assert path == GEMM and split > 1 and split * M * N * 4 <= 40 << 20, (N, K, M)
+            elif n == 4:
+                assert path == GEMM and split == 1, (N, K, M)
+            else:
+                assert path in (STRIP, TILES), (N, K, M)
+
+
 @pytest.mark.parametrize("shape,path", [
     # few rows of many columns in a format with fewer strip shapes: no search for tiles may come up empty
     ((200, 248320, 2048, 3, 32, 0, 1), GEMM), ((384, 151936, 2048, 3, 32, 0, 1), GEMM), ((384, 151936, 2048, 2, 64, 1, 1), GEMM),
