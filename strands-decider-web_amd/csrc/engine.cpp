@@ -495,7 +495,7 @@ int ha_create(const ha_config* cfg, int device, ha_engine** out) {
       e->need_gqa = slots * ha::gqa_part_slot_bytes();
       if ((rc = grow(e->scratch->gqa_part, e->need_gqa))) return bail(rc);
     }
-    e->need_gqa_rows = ha::gqa_rows_bytes((int)B * c.HK, c.max_ctx);
+    e->need_gqa_rows = ha::gqa_rows_bytes((int)B * c.HK, c.max_ctx, e->gqa_split > 0);
     e->need_gqa_marks = ha::gqa_rows_marks((int)B * c.HK, c.max_ctx) * sizeof(unsigned);
     if ((rc = grow_rows(*e->scratch, e->need_gqa_rows, e->need_gqa_marks))) return bail(rc);
     if (hipMemcpy(e->rope, rope.data(), rope.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess)
@@ -808,7 +808,7 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
       a.split = e->gqa_split; a.part_slots = e->gqa_part_slots; a.part = static_cast<float*>(sc.gqa_part.p);
       a.rows = sc.gqa_rows.p; a.rows_bytes = sc.gqa_rows.bytes;
       a.row_marks = static_cast<unsigned*>(sc.gqa_marks.p); a.marks_bytes = sc.gqa_marks.bytes;
-      const bool rows = ha::gqa_rows_takes(a);
+      const bool rows = ha::gqa_rows_takes(a) && ha::gqa_rows_faster(a);
       if (a.split > 0 && !rows) {
         // a fresh mark per launch; if the counter wraps, the marks (and partials) are cleared first
         if (++sc.gqa_epoch == 0) {

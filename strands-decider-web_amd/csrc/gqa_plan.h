@@ -43,23 +43,48 @@ __host__ __device__ inline RowsLayout rows_layout(const GqaArgs& a) {
 
 }  // namespace gqa_rows
 
-// The longest call taken, rows a sequence. gqa_attn_kernel has one workgroup per 64 rows and pair (pieces of 8 tiles in
-// engines of one or two pairs), so it catches up as rows and pairs fill the chip; the lines lie where it does. Measured at
-// 0 to 3000 cached keys, its time over this one's: 2 pairs 1.02 .. 2.6 at up to 256 rows (0.99 .. 1.02 at 400); 4 to 16
-// pairs 1.02 .. 3.1 at up to 128; 32 pairs 1.00 .. 1.5 at up to 64 but 0.5 .. 1.0 at 128; 64 pairs 0.5 .. 1.1 at any.
+// The longest call taken, rows a sequence (gqa_rows_faster: which of them are served).
 inline int gqa_rows_max(int pairs) { return pairs <= 2 ? 256 : pairs <= 16 ? 128 : pairs <= 32 ? 64 : 0; }
 
-// Marks and scratch bytes an engine holds. The scratch is what its longest short call on a full context needs, but no more
-// than one layer's K/V cache, or 64 MiB: calls that would need more are gqa_attn_kernel's (8 sequences of 4096 positions:
-// above 102 rows on a full context).
+// Whether the short-call kernels are expected to be the faster ones. gqa_attn_kernel has one workgroup per 64 rows and pair
+// that walks the key tiles, so its time hardly depends on the pairs; here every tile is a workgroup, which also replays the
+// maxima of the tiles before it, so the time grows with pairs x groups x tiles and, in long contexts, with their square.
+// Measured, gqa_attn_kernel's time over this one's, f16 rows, at 300 / 3000 / 12000 / 48000 cached keys:
+//   4 pairs   1 row 1.28 / 2.68 / 3.04 / 2.67   64 rows 2.38 / 3.06 / 3.42 / 2.60   128 rows 2.40 / 2.40 / 2.52 / 1.59
+//   16 pairs  1 row 1.27 / 1.96 / 1.84 / 1.18   64 rows 2.24 / 1.83 / 1.52 / 1.00   128 rows 1.53 / 1.04 / 0.78 / 0.49
+//   32 pairs  1 row 1.28 / 1.42 / 1.13 / 0.69   64 rows 1.49 / 0.99 / 0.78 / 0.48
+//   2 pairs, whose key ranges are split: 1 row 1.30 / 1.25 / 1.15 / 1.04 (96000: 0.97)   64 rows 2.40 / 2.23 / 1.58 / 1.18 (0.94)
+//             128 rows 2.42 / 1.64 / 1.12 / 0.82   256 rows 2.61 / 1.03 / 0.66 / 0.42
+inline bool gqa_rows_faster(int pairs, bool split, int L, int nt) {
+  const int ngrp = (L + gqa_rows::kG - 1) / gqa_rows::kG;
+  if (split) {
+    constexpr int kTiles[8] = {1200, 1200, 750, 300, 150, 80, 65, 55};  // by row groups: the tiles up to which this is the faster
+    return ngrp <= 8 && nt <= kTiles[ngrp - 1];
+  }
+  // ns: 45 a workgroup and 0.055 more for each tile of the context, against 1700 a tile (2800 with both 32-row halves; a few rows
+  // cost this side less too) and 12000 that the launches and the K/V rows take less
+  return (double)pairs * ngrp * (45.0 + 0.055 * nt) * nt <= (L <= 8 ? 1850.0 : L <= 32 ? 1700.0 : 2800.0) * nt + 12000.0;
+}
+inline bool gqa_rows_faster(const GqaArgs& a) { return gqa_rows_faster(a.B * a.HK, a.split > 0, a.L, gqa_rows::rows_layout(a).nt); }
+
+// Marks and scratch bytes an engine holds: what the calls need that gqa_rows_faster serves. (8 sequences of 4096 positions 66 MB
+// beside 67 MB of K/V a layer, of 32768 336 beside 537 MB; four pairs at most 1.25 times a layer's K/V.)
 inline size_t gqa_rows_marks(int pairs, int max_ctx) {
   return (size_t)pairs * ((gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG) * ((max_ctx + gqa_rows::kTile - 1) / gqa_rows::kTile);
 }
-inline size_t gqa_rows_bytes(int pairs, int max_ctx) {
-  const size_t groups = (gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG;
-  const size_t halves = 2 * (size_t)((max_ctx + gqa_rows::kTile - 1) / gqa_rows::kTile);
-  const size_t all = pairs * groups * 4 * halves * gqa_rows::kUnitBytes, cache = (size_t)pairs * max_ctx * 256 * 2 * 2;
-  return std::min(all, std::max(cache, (size_t)64 << 20));
+inline size_t gqa_rows_bytes(int pairs, int max_ctx, bool split) {
+  size_t units = 0;
+  const int all = (max_ctx + gqa_rows::kTile - 1) / gqa_rows::kTile;
+  for (int L = gqa_rows::kG; L <= gqa_rows_max(pairs); L += gqa_rows::kG) {
+    int lo = 0, hi = all;  // the most tiles served: more rows or tiles never make it the faster again
+    while (lo < hi) {
+      const int nt = (lo + hi + 1) / 2;
+      if (gqa_rows_faster(pairs, split, L, nt)) lo = nt;
+      else hi = nt - 1;
+    }
+    units = std::max(units, (size_t)pairs * (L / gqa_rows::kG) * 4 * 2 * lo);
+  }
+  return units * gqa_rows::kUnitBytes;
 }
 
 // Whether launch_gqa_rows can run a call: its shape (as launch_gqa checks it), and its scratch, which may be missing or too
