@@ -75,14 +75,14 @@ inline size_t gqa_rows_marks(int pairs, int max_ctx) {
 inline size_t gqa_rows_bytes(int pairs, int max_ctx, bool split) {
   size_t units = 0;
   const int all = (max_ctx + gqa_rows::kTile - 1) / gqa_rows::kTile;
-  for (int L = gqa_rows::kG; L <= gqa_rows_max(pairs); L += gqa_rows::kG) {
+  for (int L = 8; L <= gqa_rows_max(pairs); L = L == 8 ? gqa_rows::kG : L + gqa_rows::kG) {
     int lo = 0, hi = all;  // the most tiles served: more rows or tiles never make it the faster again
     while (lo < hi) {
       const int nt = (lo + hi + 1) / 2;
       if (gqa_rows_faster(pairs, split, L, nt)) lo = nt;
       else hi = nt - 1;
     }
-    units = std::max(units, (size_t)pairs * (L / gqa_rows::kG) * 4 * 2 * lo);
+    units = std::max(units, (size_t)pairs * ((L + gqa_rows::kG - 1) / gqa_rows::kG) * 4 * 2 * lo);
   }
   return units * gqa_rows::kUnitBytes;
 }
