@@ -22,7 +22,8 @@
 // that many per head); a longer call is several launches, the state carried between them in S_out.
 // Bound: a chain of memory round trips (state and rows in, raw outputs out, counter, raw outputs back). Off that chain since:
 // z and the gains are loaded before the first token instead of after the hand-off, the state is stored after the hand-off
-// instead of before it, and only where a snapshot (or the next launch) reads it. One row, 8 sequences after 1536: 9.6 ->
+// instead of before it, and only where a snapshot (or the next launch) reads it (z and the gains only in launches of few
+// workgroups, see launch_gdn_sequential). One row, 8 sequences after 1536: 9.6 ->
 // 7.4 us a launch without, 8 MB of state less written.
 #include "ha_kernels.h"
 
@@ -84,8 +85,9 @@ __device__ __forceinline__ f4 ld_dev4(const float* base, int off_bytes) {
   return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, off_bytes, 0, 16));
 }
 
-// rows [r0, r1) of the call (absolute positions; outputs for rows >= P), one launch; keep: store the state after them
-template <typename T>
+// rows [r0, r1) of the call (absolute positions; outputs for rows >= P), one launch; keep: store the state after them;
+// kEarly: the gated norm's factors loaded before the first token
+template <typename T, bool kEarly>
 __global__ __launch_bounds__(256) void gdn_seq_kernel(GdnArgs a, int r0, int r1, bool keep) {
   const int bh = blockIdx.x / kGroups, g = blockIdx.x % kGroups;
   const int b = bh / a.H, h = bh % a.H;
@@ -201,18 +203,20 @@ __global__ __launch_bounds__(256) void gdn_seq_kernel(GdnArgs a, int r0, int r1,
   load_row(r0, x0, a0, b0);
   load_row(r0 + 1, x1, a1, b1);
   // the gated norm's z and gains (4 threads per output row, 32 columns each; at most 64 rows), whichever workgroup of the
-  // head comes to use them: loaded now, they are off the path after the last token
+  // head comes to use them: loaded before the first token they are off the path after the last one, but take 64 registers
+  // (190 against 126: two workgroups a CU instead of four)
   const int nrows = r1 - orow0, nt = tid >> 2, nc0 = 32 * (tid & 3);
   const bool norms = a.gnorm && nt < nrows;
   float z[32], gw[32];
-  if (norms) {
+  auto load_norm = [&]() {
     const T* zrow = static_cast<const T*>(a.in) + ((size_t)b * a.L + (orow0 + nt - a.P)) * a.stride + a.C + h * kDV + nc0;
 #pragma unroll
     for (int c = 0; c < 32; c++) {
       z[c] = (float)zrow[c];
       gw[c] = a.gnorm[nc0 + c];
     }
-  }
+  };
+  if (kEarly && norms) load_norm();
   for (int r = r0; r < r1; r += 2) {
     step(r, x0, a0, b0);
     if (r + 1 < r1) step(r + 1, x1, a1, b1);
@@ -239,6 +243,7 @@ __global__ __launch_bounds__(256) void gdn_seq_kernel(GdnArgs a, int r0, int r1,
   store_state();
   __syncthreads();
   if (!last || !norms) return;
+  if (!kEarly) load_norm();
   f4 v[8];
   float ss = 0.0f;
 #pragma unroll
@@ -270,10 +275,13 @@ hipError_t launch_gdn_sequential(const GdnArgs& a, hipStream_t s) {
   for (int r0 = a.s0; r0 < end;) {
     const int r1 = min(end, max(r0, a.P) + kSegRows);
     const bool keep = a.keep_state || r1 < end;  // the next launch continues from it
-    if (a.dtype == 0)
-      hipLaunchKernelGGL(gdn_seq_kernel<float>, grid, block, 0, s, a, r0, r1, keep);
-    else
-      hipLaunchKernelGGL(gdn_seq_kernel<_Float16>, grid, block, 0, s, a, r0, r1, keep);
+    // up to 512 workgroups (8 sequences of 16 heads) two a CU hold them all: the early loads cost nothing and take 0.3 us off a
+    // step (8 sequences 8.4 -> 8.1 us); beyond, four a CU count for more (16 sequences 12.1 -> 9.4 us, 32 22.1 -> 15.7,
+    // 64 rows of 32 332 -> 275)
+    const bool early = grid.x <= 512;
+    auto k = a.dtype == 0 ? (early ? gdn_seq_kernel<float, true> : gdn_seq_kernel<float, false>)
+                          : (early ? gdn_seq_kernel<_Float16, true> : gdn_seq_kernel<_Float16, false>);
+    hipLaunchKernelGGL(k, grid, block, 0, s, a, r0, r1, keep);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     r0 = r1;

@@ -58,3 +58,24 @@ def test_sequential_prefix_suffix_bit_exact(P, L):
     np.testing.assert_array_equal(pre, full[:, :P])
     np.testing.assert_array_equal(suf, full[:, P:])
     np.testing.assert_array_equal(_state(ssnap, 2), _state(fsnap, 2))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("T", [1, 2, 63, 66, 131])
+def test_many_sequences_equal_few(T, f16):
+    # launches of more than 512 workgroups (9 sequences of 16 heads) load the gated norm's factors after the last token: the
+    # same rows as in an engine of 3 sequences, and for one of them the oracle's
+    B, dt = 9, np.float16 if f16 else np.float32
+    x, p = gdn_inputs(T, B, seed=4, dtype=dt), synth.gdn_params(seed=4)
+    many, few = (Runner(["linear_attention"], batch=b, lin_dtype=ha.F16 if f16 else ha.F32) for b in (B, 3))
+    for r in (many, few):
+        r.set_params(0, p)
+    (out,), _ = many.forward([x], recurrence=ha.SEQUENTIAL)
+    for b in range(0, B, 3):
+        (o,), _ = few.forward([x[b:b + 3]], recurrence=ha.SEQUENTIAL)
+        if f16:  # (a product's last rounding, f32 first or not, is the compiler's choice: one unit of an f16 result)
+            np.testing.assert_allclose(out[b:b + 3], o, rtol=2 ** -10, atol=1e-7)
+        else:
+            np.testing.assert_array_equal(out[b:b + 3], o)
+    ref, _ = oracle_gdn(x[8:9].astype(np.float32), p)
+    assert rel_err(out[8:9], ref) < (1e-2 if f16 else TOL)
