@@ -753,6 +753,7 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
   };
   auto add_tail = [&](int i) {
     t.in[t.n] = layer_in[i]; t.tail[t.n] = resume ? resume->layers[i].tail : sc.zeros.p; t.tail_out[t.n] = kept.s->layers[i].tail;
+    t.state[t.n] = e->layers[i].S; t.state_out[t.n] = kept.s->layers[i].S;
     t.n++;
     return t.n == ha::kTailLayers ? flush_tails() : hipSuccess;
   };
@@ -834,11 +835,9 @@ int ha_forward(ha_engine* e, int L, const void* const* layer_in, void* const* la
   }
   if (late) {
     if (int rc = allocate()) return rc;
-    for (int i = 0; i < c.n_layers; i++) {
-      if (e->layers[i].kind != HA_LINEAR_ATTENTION) continue;
-      HA_HIP(hipMemcpyAsync(kept.s->layers[i].S, e->layers[i].S, state_bytes, hipMemcpyDeviceToDevice, st));
-      HA_HIP(add_tail(i));
-    }
+    t.state_bytes = state_bytes;
+    for (int i = 0; i < c.n_layers; i++)
+      if (e->layers[i].kind == HA_LINEAR_ATTENTION) HA_HIP(add_tail(i));
   }
   if (const hipError_t he = flush_tails(); he != hipSuccess)
     return fail(HA_ERR_DEVICE, std::string("tail update: ") + hipGetErrorString(he));

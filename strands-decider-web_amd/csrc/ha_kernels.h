@@ -104,6 +104,9 @@ struct TailArgs {
   const void* in[kTailLayers];    // per layer: the call's input rows, [B][L][stride]
   const void* tail[kTailLayers];  // per layer: the raw-row tail the call resumed from, [B][tail_cap_in][stride]
   void* tail_out[kTailLayers];    // per layer: the snapshot's raw-row tail, [B][tail_cap_out][stride]
+  size_t state_bytes = 0;         // of a layer's state, where the layers' states are copied too
+  const void* state[kTailLayers];
+  void* state_out[kTailLayers];
 };
 
 hipError_t launch_gdn_sequential(const GdnArgs& a, hipStream_t s);

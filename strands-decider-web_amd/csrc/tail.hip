@@ -34,6 +34,13 @@ struct alignas(16) U16 {
   unsigned w[4];
 };
 
+// The layers' states into a snapshot whose memory came after their launches: grid (blocks, layers), 16 bytes a thread and step.
+__global__ __launch_bounds__(256) void state_copy_kernel(TailArgs a) {
+  const U16* s = static_cast<const U16*>(a.state[blockIdx.y]);
+  U16* d = static_cast<U16*>(a.state_out[blockIdx.y]);
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < a.state_bytes / 16; i += (size_t)gridDim.x * 256) d[i] = s[i];
+}
+
 template <typename T>
 hipError_t launch_typed(const TailArgs& a, int rows, hipStream_t s) {
   constexpr int per = 16 / sizeof(T);
@@ -53,7 +60,13 @@ hipError_t launch_typed(const TailArgs& a, int rows, hipStream_t s) {
 hipError_t launch_tail_update(const TailArgs& a, hipStream_t s) {
   const int rows = a.P + a.L - a.dst_first;
   if (rows <= 0 || a.n <= 0) return hipSuccess;
-  if (rows > a.tail_cap_out || a.n > kTailLayers) return hipErrorInvalidValue;
+  if (rows > a.tail_cap_out || a.n > kTailLayers || a.state_bytes % 16) return hipErrorInvalidValue;
+  if (a.state_bytes) {
+    const size_t steps = (a.state_bytes / 16 + 255) / 256;
+    hipLaunchKernelGGL(state_copy_kernel, dim3((unsigned)(steps < 512 ? steps : 512), a.n), dim3(256), 0, s, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   return a.dtype == 0 ? launch_typed<float>(a, rows, s) : launch_typed<_Float16>(a, rows, s);
 }
 

@@ -69,6 +69,7 @@ size_t gdn_split_image_bytes() { return 1024; }
 hipError_t launch_tail_update(const TailArgs& a, hipStream_t) {
   calls.push_back("tails");
   for (int i = 0; i < a.n; i++) memset(a.tail_out[i], 7, 64);
+  for (int i = 0; i < a.n && a.state_bytes; i++) memcpy(a.state_out[i], a.state[i], a.state_bytes);
   return hipSuccess;
 }
 hipError_t launch_gqa(const GqaArgs& a, hipStream_t) { calls.push_back("gqa"); gqa_calls.push_back(a); return hipSuccess; }
