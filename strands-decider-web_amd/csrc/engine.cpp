@@ -495,7 +495,7 @@ int ha_create(const ha_config* cfg, int device, ha_engine** out) {
       e->need_gqa = slots * ha::gqa_part_slot_bytes();
       if ((rc = grow(e->scratch->gqa_part, e->need_gqa))) return bail(rc);
     }
-    e->need_gqa_rows = ha::gqa_rows_bytes((int)B * c.HK, c.max_ctx, e->gqa_split > 0);
+    e->need_gqa_rows = ha::gqa_rows_bytes((int)B * c.HK, c.max_ctx, e->gqa_split > 0, c.full_dtype == HA_F32);
     e->need_gqa_marks = ha::gqa_rows_marks((int)B * c.HK, c.max_ctx) * sizeof(unsigned);
     if ((rc = grow_rows(*e->scratch, e->need_gqa_rows, e->need_gqa_marks))) return bail(rc);
     if (hipMemcpy(e->rope, rope.data(), rope.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess)

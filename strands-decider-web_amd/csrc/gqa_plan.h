@@ -55,31 +55,39 @@ inline int gqa_rows_max(int pairs) { return pairs <= 2 ? 256 : pairs <= 16 ? 128
 //   32 pairs  1 row 1.28 / 1.42 / 1.13 / 0.69   64 rows 1.49 / 0.99 / 0.78 / 0.48
 //   2 pairs, whose key ranges are split: 1 row 1.30 / 1.25 / 1.15 / 1.04 (96000: 0.97)   64 rows 2.40 / 2.23 / 1.58 / 1.18 (0.94)
 //             128 rows 2.42 / 1.64 / 1.12 / 0.82   256 rows 2.61 / 1.03 / 0.66 / 0.42
-inline bool gqa_rows_faster(int pairs, bool split, int L, int nt) {
+// f32 rows are read directly by every tile's workgroup, twice (16 pairs, 3000 keys: 1 row 1.77, 32 rows 1.17, 64 rows 1.18, 96
+// rows 0.74; 32 pairs: 1.21, 0.73, 0.61; an empty context: 32 rows 0.82 .. 0.85).
+inline bool gqa_rows_faster(int pairs, bool split, bool f32, int L, int nt) {
   const int ngrp = (L + gqa_rows::kG - 1) / gqa_rows::kG;
-  if (split) {
-    constexpr int kTiles[8] = {1200, 1200, 750, 300, 150, 80, 65, 55};  // by row groups: the tiles up to which this is the faster
-    return ngrp <= 8 && nt <= kTiles[ngrp - 1];
+  const bool some = f32 && L > 8;  // f32 rows whose loads count
+  if (split) {  // by row groups: the tiles up to which this is the faster
+    constexpr int kTiles[8] = {1200, 1200, 750, 300, 150, 80, 65, 55}, kTiles32[8] = {150, 350, 150, 90, 60, 35, 30, 25};
+    return ngrp <= 8 && nt <= (some ? kTiles32 : f32 ? kTiles + 3 : kTiles)[ngrp - 1] && !(some && ngrp == 1 && nt < 3);
   }
-  // ns: 45 a workgroup and 0.055 more for each tile of the context, against 1700 a tile (2800 with both 32-row halves; a few rows
-  // cost this side less too) and 12000 that the launches and the K/V rows take less
-  return (double)pairs * ngrp * (45.0 + 0.055 * nt) * nt <= (L <= 8 ? 1850.0 : L <= 32 ? 1700.0 : 2800.0) * nt + 12000.0;
+  const double wg = (double)pairs * ngrp * nt, replay = 0.055 * nt * wg;  // ns, as below
+  if (some)  // the chip takes 192 such workgroups in one go
+    return 27000.0 + 250.0 * nt + 75.0 * std::max(0.0, wg - 192.0) + replay <= (L <= 32 ? 21000.0 + 1680.0 * nt : 33000.0 + 2570.0 * nt);
+  // 45 ns a workgroup and 0.055 more for each tile of the context, against 1700 a tile (2800 with both 32-row halves; a few
+  // rows cost this side less too) and 12000 that the launches and the K/V rows take less
+  return 45.0 * wg + replay <= (L <= 8 ? 1850.0 : L <= 32 ? 1700.0 : 2800.0) * nt + 12000.0;
 }
-inline bool gqa_rows_faster(const GqaArgs& a) { return gqa_rows_faster(a.B * a.HK, a.split > 0, a.L, gqa_rows::rows_layout(a).nt); }
+inline bool gqa_rows_faster(const GqaArgs& a) {
+  return gqa_rows_faster(a.B * a.HK, a.split > 0, a.dtype == 0, a.L, gqa_rows::rows_layout(a).nt);
+}
 
 // Marks and scratch bytes an engine holds: what the calls need that gqa_rows_faster serves. (8 sequences of 4096 positions 66 MB
 // beside 67 MB of K/V a layer, of 32768 336 beside 537 MB; four pairs at most 1.25 times a layer's K/V.)
 inline size_t gqa_rows_marks(int pairs, int max_ctx) {
   return (size_t)pairs * ((gqa_rows_max(pairs) + gqa_rows::kG - 1) / gqa_rows::kG) * ((max_ctx + gqa_rows::kTile - 1) / gqa_rows::kTile);
 }
-inline size_t gqa_rows_bytes(int pairs, int max_ctx, bool split) {
+inline size_t gqa_rows_bytes(int pairs, int max_ctx, bool split, bool f32) {
   size_t units = 0;
   const int all = (max_ctx + gqa_rows::kTile - 1) / gqa_rows::kTile;
   for (int L = 8; L <= gqa_rows_max(pairs); L = L == 8 ? gqa_rows::kG : L + gqa_rows::kG) {
-    int lo = 0, hi = all;  // the most tiles served: more rows or tiles never make it the faster again
+    int lo = std::min(all, 4), hi = all;  // the most tiles served: beyond a few, more tiles never make it the faster again
     while (lo < hi) {
       const int nt = (lo + hi + 1) / 2;
-      if (gqa_rows_faster(pairs, split, L, nt)) lo = nt;
+      if (gqa_rows_faster(pairs, split, f32, L, nt)) lo = nt;
       else hi = nt - 1;
     }
     units = std::max(units, (size_t)pairs * ((L + gqa_rows::kG - 1) / gqa_rows::kG) * 4 * 2 * lo);

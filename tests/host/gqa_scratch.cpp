@@ -16,14 +16,16 @@ int main() {
   const size_t big = ~(size_t)0;
   for (int pairs : {1, 2, 4, 8, 16, 32, 64})
     for (int ctx : {64, 4096, 32768, 262144, 1 << 20})
-      CHECK(gqa_rows_bytes(pairs, ctx, pairs <= 2) <= std::max((size_t)24 << 20, (size_t)pairs * ctx * 256 * 5));
+      CHECK(gqa_rows_bytes(pairs, ctx, pairs <= 2, false) <= std::max((size_t)24 << 20, (size_t)pairs * ctx * 256 * 5));
   // every call that the short-call kernels are expected to be the faster for fits the engine's scratch
-  for (int B : {1, 2, 3, 5, 8, 16})
+  for (int f16 = 0; f16 < 2; f16++)
+   for (int B : {1, 2, 3, 5, 8, 16})
     for (int ctx : {64, 2048, 4096, 32768, 131072}) {
-      const size_t n = gqa_rows_bytes(2 * B, ctx, B == 1), m = ha::gqa_rows_marks(2 * B, ctx) * 4;
+      const size_t n = gqa_rows_bytes(2 * B, ctx, B == 1, !f16), m = ha::gqa_rows_marks(2 * B, ctx) * 4;
       for (int L = 1; L <= ha::gqa_rows_max(2 * B) && L <= ctx; L++)
         for (int P = 0; P + L <= ctx; P += 63 + (P >> 5)) {
           ha::GqaArgs x = args(B, 2, P, L, ctx, n, m);
+          x.dtype = f16;
           x.split = B == 1 ? std::max(8, (ctx / 64 + 7) / 8) : 0;
           if (ha::gqa_rows_faster(x)) CHECK(ha::gqa_rows_takes(x));
         }
@@ -51,6 +53,14 @@ int main() {
   CHECK(faster(8, 1500, 128, 0) && !faster(8, 12000, 128, 0) && faster(16, 12000, 1, 0) && !faster(16, 12000, 32, 0) && !faster(16, 24000, 1, 0));
   CHECK(faster(16, 1500, 64, 0) && !faster(16, 6000, 64, 0) && faster(2, 96000, 128, 0) && faster(3, 48000, 128, 0));
   CHECK(faster(1, 48000, 1, 100) && !faster(1, 96000, 64, 200) && faster(1, 12000, 128, 25) && !faster(1, 24000, 128, 50));
+  auto faster32 = [&](int B, int P, int L, int split) {
+    ha::GqaArgs x = args(B, 2, P, L, 1 << 20, big, big);
+    x.split = split; x.dtype = 0;
+    return ha::gqa_rows_faster(x);
+  };
+  CHECK(faster32(8, 3000, 64, 0) && !faster32(8, 3000, 96, 0) && !faster32(16, 3000, 32, 0) && faster32(16, 3000, 1, 0));
+  CHECK(!faster32(8, 0, 32, 0) && faster32(8, 300, 32, 0) && !faster32(1, 0, 16, 8) && faster32(1, 300, 16, 8));
+  CHECK(faster32(1, 3000, 128, 8) && !faster32(1, 12000, 128, 25) && !faster32(1, 3000, 256, 8) && faster32(1, 300, 256, 8));
   CHECK(faster(1, 1500, 256, 8) && faster(1, 3000, 256, 8) && !faster(1, 6000, 256, 13) && !faster(1, 6000, 192, 13));
 
   // an engine is made where its caches fit and the scratch does not; its short calls then run the general kernel
@@ -60,7 +70,7 @@ int main() {
   const void* ins[1] = {in};
   void* outs[1] = {out};
   ha_engine *e = nullptr, *f = nullptr;
-  limit = gqa_rows_bytes(2, 4096, true) - 1;  // (18 MB; the cache is 8)
+  limit = gqa_rows_bytes(2, 4096, true, false) - 1;  // (18 MB; the cache is 8)
   CHECK(ha_create(&c, 0, &e) == HA_OK);
   CHECK(ha_forward(e, 64, ins, outs, nullptr, nullptr, nullptr) == HA_OK && calls.back() == "gqa");
   // joining another engine's set, and leaving it, likewise
@@ -69,7 +79,7 @@ int main() {
   CHECK(ha_forward(f, 64, ins, outs, nullptr, nullptr, nullptr) == HA_OK && calls.back() == "gqa_rows");
   void* st = nullptr;
   CHECK(ha_get_stream(f, &st) == HA_OK && ha_set_stream(e, st) == HA_OK);
-  limit = gqa_rows_bytes(2, 4096, true) - 1;
+  limit = gqa_rows_bytes(2, 4096, true, false) - 1;
   CHECK(ha_share_scratch(e, f) == HA_OK);
   CHECK(ha_forward(e, 64, ins, outs, nullptr, nullptr, nullptr) == HA_OK && calls.back() == "gqa_rows");
   CHECK(ha_set_stream(e, nullptr) == HA_OK);
