@@ -103,9 +103,9 @@ typedef struct ha_forward_opts {
                       computed on. Implies a wait, like layer_ms */
   int debug_unpublished_waits; /* test only, 0 otherwise. No counterpart in the reference. 1: every bounded
                       cross-workgroup wait of this call (the paired form's tile-set wait, the split form's
-                      packed-state wait, the split-key attention merge, a short attention call's maxima) waits for a value no workgroup of it
-                      publishes, for a few polls each, then goes on; every kernel still ends, the outputs are
-                      undefined, and the failure is reported as HA_ERR_DEVICE (exercises that path from the host) */
+                      packed-state wait, the split-key attention merge, a short attention call's maxima) waits for a
+                      value no workgroup of it publishes, for a few polls each, then goes on; every kernel still
+                      ends, the outputs are undefined, and the failure is reported as HA_ERR_DEVICE (exercises that path from the host) */
 } ha_forward_opts;
 
 const char* ha_last_error(void);
@@ -115,8 +115,10 @@ int ha_abi_version(void);
    no HIP device is visible. */
 int ha_device_arch(int device, char* name, size_t bytes);
 
-/* Engine.create / constructor (engine.js:63-111): validates the config, allocates the working state, history
-   and K/V buffers and the RoPE table on HIP device `device`, and creates the engine's stream. */
+/* Engine.create / constructor (engine.js:63-111): validates the config, allocates the working state and K/V buffers,
+   the RoPE table and the buffers that calls work in on HIP device `device`, and creates the engine's stream. (The
+   scratch of short full-attention calls is optional: without the memory for it the general kernel serves them, with
+   the same results.) */
 int ha_create(const ha_config* cfg, int device, ha_engine** out);
 int ha_destroy(ha_engine* e);
 
@@ -126,8 +128,8 @@ int ha_destroy(ha_engine* e);
    so that engines holding one set always run on one stream. */
 int ha_set_stream(ha_engine* e, void* stream);
 /* Let engine e use the call-time device buffers of `holder` (chunk images, the sequential form's raw outputs and
-   counters, split-GQA partials, the zero history), growing them to what e's shape needs, and free e's own set once
-   nothing else holds it. For the per-layer engines of one torso on one stream: their calls then run one after
+   counters, split-GQA partials, short attention calls' scratch and marks, the zero history), growing them to what
+   e's shape needs, and free e's own set once nothing else holds it. For the per-layer engines of one torso on one stream: their calls then run one after
    another and one set serves all of them. Both engines must already run on one stream (HA_ERR_ARG otherwise), and
    ha_set_stream keeps it so. The set lives until the last engine holding it is destroyed. No counterpart in the
    reference, whose engine holds one set of buffers for all its layers (engine.js:89-107). Waits for the device to

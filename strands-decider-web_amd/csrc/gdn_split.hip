@@ -68,7 +68,8 @@ __device__ __forceinline__ h8 join(const f4& lo, const f4& hi) { return pack_b(l
 // are then spread over the four waves and written to the image straight from registers.
 // 8 waves: wave w + 4 takes half of wave w's tiles where the text below speaks of four waves, and a conv lane 4 rows
 // instead of 8. A workgroup's chain of phases is what bounds the kernel (a few workgroups a CU at most), and the wide ones
-// halve; per element the arithmetic is the same. 4 waves of 8 rows -> this, us a layer: 61 rows after 1531 (B = 1) 25.3 -> 23.5,
+// halve; the operations of an element are the same (f32 rows: the same bits; with f16 rows the compiler rounds a few products
+// of the tiles to f32 first or not where it did the other before, 600 of 3.1 million outputs a last bit apart). 4 waves of 8 rows -> this, us a layer: 61 rows after 1531 (B = 1) 25.3 -> 23.5,
 // B = 1, T = 1531 52.0 -> 49.9, T = 4000 104 -> 99; B = 2, T = 2048 97 -> 91.
 constexpr int kHalves = 2, kPT = 256 * kHalves;
 constexpr int kPRG = 8 / kHalves;  // rows per conv lane

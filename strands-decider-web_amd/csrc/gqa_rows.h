@@ -1,5 +1,6 @@
-// Full attention of a short call (a decode step, a resumed question), gfx950, compiled with gqa.hip: the same arithmetic as gqa.hip, row for row
-// and bit for bit, in two launches that put every key tile and every slice of output dims on a workgroup of its own.
+// Full attention of a short call (a decode step, a resumed question), gfx950, part of gqa.hip: the same arithmetic as gqa.hip, row
+// for row and bit for bit (gqa_common.h writes out the roundings the two share), in two launches that put every
+// key tile and every slice of output dims on a workgroup of its own.
 //
 // A short call has one or two 32-row query groups per (sequence, KV head), so gqa_attn_kernel has a handful of workgroups
 // that walk the key tiles one after another: 51 us for a decode step of 8 sequences at 1536 keys, 50 us for 61 rows after
@@ -18,8 +19,9 @@
 // Bound: latency (a dependent chain of launches, loads and one cross-workgroup hand-off); the K/V cache is read once.
 // Waits: a workgroup waits only for workgroups of lower index in its grid. Each XCD takes its blocks in order, so the
 // lowest unfinished block is always resident and waits for finished ones: every wait ends, and each is bounded besides.
-// Measured, f16 rows, us a call, before -> now: 61 rows after 1531 (1 sequence) 61 -> 23; one row after 1536 (8 sequences)
-// 56 -> 28 (scores 15.8, values 12.3), after 3000 93 -> 47; 64 rows of an empty context 26 -> 17.
+// Measured, f16 rows, us a call, gqa_attn_kernel -> this: 61 rows after 1531 (1 sequence) 61 -> 23 (traced: scores 12.8, values
+// 9.5); one row after 1536 (8 sequences) 56 -> 30 (18.0, 14.3), after 3000 93 -> 48; 64 rows of an empty context 27 -> 19. Where
+// it is the faster one and where not: gqa_plan.h.
 #pragma once
 #include <algorithm>
 

@@ -1,4 +1,4 @@
-// MatMulNBits projection of a few hundred rows or less, gfx950, compiled with torso.hip: y[M][N] = a[M][K] x W^T (formats: mnb.hip).
+// MatMulNBits projection of a few hundred rows or less, gfx950, part of torso.hip: y[M][N] = a[M][K] x W^T (formats: mnb.hip).
 //
 // Bound: moving a. Each workgroup needs all of its rows of a, so M x K x 2 bytes pass through the L2 once per column
 // tile; the packed weights (0.56 bytes each) are read once or twice. A wave cannot load its MFMA operands from a
@@ -19,9 +19,9 @@
 // Measured, us per call back to back, weights rotating through eight matrices, with the kernels this replaced (the
 // register-operand kernel up to 64 rows, the tiled GEMM with K split over workgroups above) -> now:
 //   N x K          M = 3       17         61          68          128         256
-//   12288 x 2048   7.7 -> 5.9  13.3->6.7  25.8->9.4   22.8->10.2  26.4->14.0  35.2->25.1
-//   2048 x 6144    7.7 -> 6.3  13.9->6.5  24.9->7.7   22.6->8.7   23.9->9.4   24.9->14.7
-//   2048 x 2048    4.4 -> 4.4  5.9 ->4.4  9.8 ->4.5   13.8->4.7   14.6->4.9   16.6->6.5
+//   12288 x 2048   7.5 -> 5.7  13.3->6.4  25.8->9.1   22.1->9.9   25.8->13.5  35.4->25.1
+//   2048 x 6144    7.7 -> 6.3  13.9->6.3  25.0->7.5   21.7->8.5   23.1->9.3   24.6->14.7
+//   2048 x 2048    4.0 -> 3.8  5.8 ->3.9  9.8 ->4.2   13.7->4.4   14.3->4.5   15.8->6.1
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -1,4 +1,4 @@
-// MatMulNBits projection of many rows with 4-bit weights, gfx950, compiled with mnb.hip: y[M][N] = a[M][K] x W^T on
+// MatMulNBits projection of many rows with 4-bit weights, gfx950, part of mnb.hip: y[M][N] = a[M][K] x W^T on
 // matrix-core tiles.
 //
 // Bound: the matrix cores and, beside them, LDS reads. mnb_gemm_kernel dequantises a weight tile into LDS, so each MFMA
@@ -14,13 +14,14 @@
 // in whole rounds, and the rest to the smaller tiles (plan_tiles). An N just over a multiple of 256 (8256 = 32 x 256 + 64)
 // would buy a round for its last columns: those go to the strip kernel.
 //
-// Measured, us a call, weights rotating through eight matrices, mnb_gemm_kernel -> this (or the strip
+// Measured, us a call over a long run of calls, weights rotating through eight matrices, mnb_gemm_kernel -> this (or the strip
 // kernel where that is the faster, *):
 //   N x K          M = 333     512         1024        1531        2048
-//   12288 x 2048   43 -> 33    45 -> 35    79 -> 65    122 -> 99   132 -> 112
-//   8256 x 2048    34 -> 27*   41 -> 29    78 -> 46    79 -> 70    121 -> 83
-//   2048 x 6144    29 -> 20*   34 -> 24*   52 -> 45*   70 -> 57    78 -> 65
-//   5120 x 2048    27 -> 17*   33 -> 22    43 -> 32    49 -> 39    78 -> 60
+//   12288 x 2048   42 -> 31    44 -> 34    79 -> 65    122 -> 102  135 -> 114
+//   8256 x 2048    34 -> 27*   41 -> 29    79 -> 45    80 -> 71    122 -> 85
+//   2048 x 6144    28 -> 20*   33 -> 24*   52 -> 45*   70 -> 58    78 -> 68
+//   5120 x 2048    26 -> 17*   32 -> 22    43 -> 32    49 -> 40    79 -> 60
+// In a run of 20 calls of one matrix (HIP events; a kernel trace agrees) M = 2048 takes 124, 92, 77 and 69: the clock differs.
 #pragma once
 #include <hip/hip_runtime.h>
 
